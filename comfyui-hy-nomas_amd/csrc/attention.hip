@@ -27,6 +27,14 @@
 // 16 different bank quads).  The direct loads write 1 KB per wave instruction in lane order, so the swizzle
 // is applied on the global side (the lane fetches the logical chunk of its physical slot).
 //
+// Key segments.  The keys of a query are the concatenation of up to three segments, read where they lie: up to two
+// shared ones (the history cache and the current tokens, each with its own strides) and the text keys of the
+// query's group.  Every segment starts a new 64-key tile, and its last tile is masked, so nothing is joined in
+// memory first; V^T holds the segments one after another, each padded to whole tiles (attention_pack_kernel).  All
+// groups share one launch, which fills the chip where one group would not.  Joining, gathering and transposing per
+// group took two thirds of such a call: 24 heads, 3520 + 200 tokens over 15840 history keys in three groups went
+// from 2595 to 941 us; 16 heads x 26656 tokens, where only the V^T pass is new, from 5777 to 5448 us.
+//
 // Lazy rescale.  The running reference max m moves only when a tile's max exceeds it by more than 8 (base-2
 // units), so the probabilities exp2(s - m) stay below 2^8 and the accumulators are rescaled only a few times
 // per query instead of whenever the max grows.  The result is the same quotient: numerator and denominator
@@ -49,19 +57,40 @@ constexpr int kVTile = kHeadDim * kBK * 2;      // 16 KB
 constexpr int kAttnStage = kKTile + kVTile;
 constexpr float kSlack = 8.0f;                  // headroom of the lazy max (base-2 units)
 
+constexpr int kMaxGroups = 64;                  // query groups of one launch (the table rides in the kernel arguments)
+
+// One shared key segment: key j of batch b, head h at k + b skb + h skh + j skj, V^T position vpos + j.
+struct AttnSeg {
+  const uint16_t* k;
+  int64_t skb, skh, skj;
+  int64_t len;
+  int64_t vpos;
+};
+
+// One query group: queries rows[q_off .. q_off + q_n), workgroups from query block qb0 on, text keys t_n at row
+// t_pos (a multiple of 64) of the packed text keys.
+struct AttnGroup {
+  int qb0, q_off, q_n, t_n, t_pos;
+};
+
 struct AttnArgs {
   const uint16_t* q;
   int64_t sqb, sqh, sqi;  // element strides of batch, head, token (dims contiguous)
-  const uint16_t* k;
-  int64_t skb, skh, skj;
+  AttnSeg seg[2];
+  int nseg;
+  const uint16_t* tk;     // packed text keys [B, H, t_rows, 128], V^T positions from tvpos on
+  int64_t t_rows, tvpos;
   const uint16_t* vt;     // V^T: element (b, h, d, key position p) at vt + b svb + h svh + d svd + p
   int64_t svb, svh, svd;
   uint16_t* o;
   int64_t sob, soh, soi;
+  const int64_t* rows;    // query rows of the groups, or null: query i is row i
+  const int* owner;       // with rows: the last group that names each row, whose result it takes
   int H;
-  int64_t Lq, Lk;
   float scale_log2;       // softmax scale times log2(e): the scores are exponentiated base 2
-  int qblocks;
+  int qblocks;            // query blocks of one (batch, head)
+  int ngroups;
+  AttnGroup group[kMaxGroups];
 };
 
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8)); }
@@ -81,49 +110,83 @@ void attention_kernel(const AttnArgs a) {
   const int h2 = lane >> 5, l32 = lane & 31;
   const int bh = blockIdx.x / a.qblocks, qb = blockIdx.x % a.qblocks;
   const int64_t b = bh / a.H, hh = bh % a.H;
+  int gi = 0;
+  while (gi + 1 < a.ngroups && qb >= a.group[gi + 1].qb0) gi++;
+  const int q_n = a.group[gi].q_n, t_n = a.group[gi].t_n;
   const uint16_t* qbase = a.q + b * a.sqb + hh * a.sqh;
-  const char* kbase = reinterpret_cast<const char*>(a.k + b * a.skb + hh * a.skh);
   const char* vbase = reinterpret_cast<const char*>(a.vt + b * a.svb + hh * a.svh);
-  const uint32_t kstride = (uint32_t)(a.skj * 2), vstride = (uint32_t)(a.svd * 2);  // bytes per key / dim row
-  const int64_t q0 = (int64_t)qb * kBQ + wave * 32;
-  const int64_t qi = q0 + l32 < a.Lq ? q0 + l32 : a.Lq - 1;
+  const uint32_t vstride = (uint32_t)(a.svd * 2);  // bytes per dim row
+  const int q0 = (qb - a.group[gi].qb0) * kBQ + wave * 32;
+  const int qi = q0 + l32 < q_n ? q0 + l32 : q_n - 1;
+  const int64_t qrow = a.rows ? a.rows[a.group[gi].q_off + qi] : qi;
 
   // the wave's 32 queries: B fragments of S^T = K Q^T for the 8 steps of 16 dims (query l32, dims 16 ks + 8 h2 ..)
   bf16x8 qf[8];
 #pragma unroll
-  for (int ks = 0; ks < 8; ks++) qf[ks] = *reinterpret_cast<const bf16x8*>(qbase + qi * a.sqi + 16 * ks + 8 * h2);
+  for (int ks = 0; ks < 8; ks++) qf[ks] = *reinterpret_cast<const bf16x8*>(qbase + qrow * a.sqi + 16 * ks + 8 * h2);
 
   // direct loads of one tile: wave w fills the 1 KB blocks w, w + 4, w + 8, w + 12 of the K tile (4 rows of
   // 256 bytes each) and of the V^T tile (8 rows of 128 bytes), each lane 16 bytes at a fixed 32-bit offset
   // from the tile's buffer descriptor (wave-uniform base: no per-lane 64-bit address arithmetic)
-  uint32_t koff[4], voff[4];
+  uint32_t koff[4], voff[4], kstride = 0;
 #pragma unroll
   for (int u = 0; u < 4; u++) {
-    const int krow = (wave + 4 * u) * 4 + lane / 16, kphys = lane % 16;
-    koff[u] = (uint32_t)krow * kstride + (uint32_t)((kphys ^ (krow & 15)) << 4);
     const int vrow = (wave + 4 * u) * 8 + lane / 8, vphys = lane % 8;
     voff[u] = (uint32_t)vrow * vstride + (uint32_t)((vphys ^ ((vrow >> 1) & 7)) << 4);
   }
-  auto issue_tile = [&](int64_t j0, int buf) {
+  // the next tile to load: its first key's address, its V^T column, and the keys from it to its segment's end
+  const char *kcur = nullptr, *vcur = nullptr;
+  int64_t left = 0;
+  int seg = -1;
+  auto next_segment = [&]() {
+    do {
+      seg++;
+      if (seg < a.nseg) {
+        const AttnSeg& sg = a.seg[seg];
+        kcur = reinterpret_cast<const char*>(sg.k + b * sg.skb + hh * sg.skh);
+        vcur = vbase + sg.vpos * 2;
+        kstride = (uint32_t)(sg.skj * 2);  // bytes per key
+        left = sg.len;
+      } else {  // the group's text keys
+        kcur = reinterpret_cast<const char*>(a.tk + ((b * a.H + hh) * a.t_rows + a.group[gi].t_pos) * kHeadDim);
+        vcur = vbase + (a.tvpos + a.group[gi].t_pos) * 2;
+        kstride = kHeadDim * 2;
+        left = t_n;
+      }
+    } while (left == 0 && seg < a.nseg);
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int krow = (wave + 4 * u) * 4 + lane / 16, kphys = lane % 16;
+      koff[u] = (uint32_t)krow * kstride + (uint32_t)((kphys ^ (krow & 15)) << 4);
+    }
+  };
+  // loads the tile at the cursor into a buffer and moves the cursor; returns the tile's keys (64, or fewer at a
+  // segment's end)
+  auto issue_tile = [&](int buf) __attribute__((always_inline)) {
     char* kt = smem + buf * kAttnStage;
     char* vt = kt + kKTile;
-    const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(kbase + j0 * kstride);
-    const __amdgpu_buffer_rsrc_t vr = buffer_rsrc(vbase + j0 * 2);
-    if (j0 + kBK <= a.Lk) {
+    const __amdgpu_buffer_rsrc_t kr = buffer_rsrc(kcur);
+    const __amdgpu_buffer_rsrc_t vr = buffer_rsrc(vcur);
+    const int here = left < kBK ? (int)left : kBK;
+    if (here == kBK) {
 #pragma unroll
       for (int u = 0; u < 4; u++) b2lds16(kr, koff[u], 0, kt + (wave + 4 * u) * 1024);
     } else {
-      // the last tile: rows past the last key re-read it (their scores are masked)
-      const int last = (int)(a.Lk - 1 - j0);
+      // a segment's last tile: rows past the last key re-read it (their scores are masked)
 #pragma unroll
       for (int u = 0; u < 4; u++) {
         const int krow = (wave + 4 * u) * 4 + lane / 16, kphys = lane % 16;
-        const int r = krow < last ? krow : last;
+        const int r = krow < here - 1 ? krow : here - 1;
         b2lds16(kr, (uint32_t)r * kstride + (uint32_t)((kphys ^ (krow & 15)) << 4), 0, kt + (wave + 4 * u) * 1024);
       }
     }
 #pragma unroll
     for (int u = 0; u < 4; u++) b2lds16(vr, voff[u], 0, vt + (wave + 4 * u) * 1024);
+    left -= here;
+    kcur += (int64_t)kBK * kstride;
+    vcur += kBK * 2;
+    if (left == 0 && seg < a.nseg) next_segment();
+    return here;
   };
 
   v16f_a oacc[4];
@@ -145,19 +208,21 @@ void attention_kernel(const AttnArgs a) {
   for (int i = 0; i < 32; i++) pv[i] = 0.0f;
   const int kswz = l32 & 15, vswz = (l32 >> 1) & 7;   // the lane's rows' swizzles (rows 32 i + l32)
 
-  const int64_t nt = (a.Lk + kBK - 1) / kBK;
+  int nt = (t_n + kBK - 1) / kBK;  // tiles of all segments
+  for (int i = 0; i < a.nseg; i++) nt += (int)((a.seg[i].len + kBK - 1) / kBK);
+  int keys = 0, keys_next = 0;     // keys of the current and of the loading tile
   // tile t in stage buffer BUF (a constant, so the buffer offset rides in the LDS reads' immediate field
   // and the lane's fragment offsets stay fixed across the loop)
-  auto tile = [&](int64_t t, auto buf_c) __attribute__((always_inline)) {
+  auto tile = [&](int t, auto buf_c) __attribute__((always_inline)) {
     constexpr int BUF = decltype(buf_c)::value;
     // tile t has landed for every wave, and every wave is done with the buffer tile t + 1 refills
     wait_vm0();
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
-    if (t + 1 < nt) issue_tile((t + 1) * kBK, BUF ^ 1);
+    keys = keys_next;
+    if (t + 1 < nt) keys_next = issue_tile(BUF ^ 1);
     const char* kt = smem + BUF * kAttnStage;
     const char* vt = kt + kKTile;
-    const int64_t j0 = t * kBK;
 
     // S^T for the tile's two 32-key blocks (interleaved): lane holds query l32, keys 32 kb + 8 (r / 4) + 4 h2 + r % 4
     v16f_a s[2];
@@ -188,10 +253,10 @@ void attention_kernel(const AttnArgs a) {
       for (int i = 0; i < 4; i++) lsum += pv[4 * ks + i];
       __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
     }
-    if (j0 + kBK > a.Lk) {  // the last tile: keys past the end take no weight
-      // register r of block kb holds key j0 + 32 kb + 8 (r / 4) + (r % 4) + 4 h2: a constant per register
+    if (keys < kBK) {  // a segment's last tile: keys past its end take no weight
+      // register r of block kb holds the tile's key 32 kb + 8 (r / 4) + (r % 4) + 4 h2: a constant per register
       // against one per-lane limit
-      const int lim = (int)(a.Lk - j0) - 4 * h2;
+      const int lim = keys - 4 * h2;
 #pragma unroll
       for (int kb = 0; kb < 2; kb++)
 #pragma unroll
@@ -258,8 +323,9 @@ void attention_kernel(const AttnArgs a) {
         }
       }
   };
-  issue_tile(0, 0);
-  for (int64_t t = 0; t < nt; t += 2) {
+  next_segment();
+  keys_next = issue_tile(0);
+  for (int t = 0; t < nt; t += 2) {
     tile(t, std::integral_constant<int, 0>());
     if (t + 1 < nt) tile(t + 1, std::integral_constant<int, 1>());
   }
@@ -268,8 +334,8 @@ void attention_kernel(const AttnArgs a) {
   // normalize and store: lane holds query l32, dims 32 db + 8 rr + 4 h2 + 0..3 in registers 4 rr .. 4 rr + 3
   const float ltot = lsum + __shfl_xor(lsum, 32);
   const float inv = 1.0f / ltot;
-  if (q0 + l32 < a.Lq) {
-    uint16_t* orow = a.o + b * a.sob + hh * a.soh + (q0 + l32) * a.soi;
+  if (q0 + l32 < q_n && (a.owner == nullptr || a.owner[qrow] == gi)) {
+    uint16_t* orow = a.o + b * a.sob + hh * a.soh + qrow * a.soi;
 #pragma unroll
     for (int db = 0; db < 4; db++)
 #pragma unroll
@@ -280,6 +346,149 @@ void attention_kernel(const AttnArgs a) {
         *reinterpret_cast<uint2*>(orow + d) = w;
       }
   }
+}
+
+// V^T of every key segment, and the packed text keys, for attention_kernel.
+//
+// One workgroup takes 64 keys (one tile of one segment) of one (batch, head): it reads the 64 rows of 256 bytes
+// whole, turns them in LDS (rows of 65 dwords, so the column reads spread over the banks) and writes 128 bytes of
+// each of the 128 V^T rows, keys past the segment's end as zeros.  HBM bound: 2 bytes read and 2 written per
+// element.  Text keys are gathered by row on the way (a few hundred rows at most), and their K rows copied to the
+// packed buffer, where the attention kernel's tile loads can take them as a segment.  46 us for 24 heads x 19600
+// keys, 5.2 TB/s; torch's permuting copy of one such V took about 400 us.
+struct PackPart {
+  const uint16_t* v;
+  int64_t svb, svh, svj;
+  int64_t len, tile0;
+};
+
+struct PackArgs {
+  PackPart part[2];       // shared segments, then the text source below
+  int nparts;
+  int64_t text_tile0, tiles;
+  const uint16_t *tk_src, *tv_src;
+  int64_t tkb, tkh, tkj, tvb, tvh, tvj;
+  const int64_t* rows;
+  int64_t text_off;       // the text rows start here in rows
+  uint16_t* vt;
+  int64_t svb, svh, svd;
+  uint16_t* tk;
+  int64_t t_rows;
+  int* owner;
+  int64_t Lq;
+  int H;
+  int ngroups;
+  AttnGroup group[kMaxGroups];
+  int t_off[kMaxGroups];  // each group's first text row, from text_off
+};
+
+constexpr int kPackThreads = 256;
+
+__global__ __launch_bounds__(kPackThreads) void attention_pack_kernel(const PackArgs a) {
+  __shared__ uint32_t rows32[kBK * 65];  // row = key, 64 dwords of dim pairs, one dword of padding
+  const int tid = threadIdx.x;
+  const int64_t tile = blockIdx.x;
+  const int64_t b = blockIdx.y / a.H, h = blockIdx.y % a.H;
+  if (tile == a.tiles) {  // one more workgroup: the group whose result each query row takes (the last naming it)
+    if (blockIdx.y != 0) return;
+    for (int64_t i = tid; i < a.Lq; i += kPackThreads) a.owner[i] = -1;
+    __threadfence();
+    __syncthreads();
+    for (int g = 0; g < a.ngroups; g++)
+      for (int i = tid; i < a.group[g].q_n; i += kPackThreads) atomicMax(&a.owner[a.rows[a.group[g].q_off + i]], g);
+    return;
+  }
+  // the tile's rows
+  const uint16_t *vsrc, *ksrc = nullptr;
+  int64_t vj, first = 0, len;
+  const int64_t* idx = nullptr;
+  int64_t kpos = 0;
+  if (tile < a.text_tile0) {
+    const PackPart& p = a.part[a.nparts > 1 && tile >= a.part[1].tile0 ? 1 : 0];
+    first = (tile - p.tile0) * kBK;
+    len = p.len - first;
+    vsrc = p.v + b * p.svb + h * p.svh + first * p.svj;
+    vj = p.svj;
+  } else {
+    kpos = (tile - a.text_tile0) * kBK;
+    int g = 0;
+    while (g + 1 < a.ngroups && kpos >= a.group[g + 1].t_pos) g++;
+    first = kpos - a.group[g].t_pos;
+    len = a.group[g].t_n - first;
+    idx = a.rows + a.text_off + a.t_off[g] + first;
+    vsrc = a.tv_src + b * a.tvb + h * a.tvh;
+    ksrc = a.tk_src + b * a.tkb + h * a.tkh;
+    vj = a.tvj;
+  }
+  const int n = len < kBK ? (int)len : kBK;
+  const int c = tid & 15;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    const int r = (tid >> 4) + 16 * u;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (r < n) {
+      const int64_t row = idx ? idx[r] : r;
+      v = ld_nt16(vsrc + row * vj + c * 8);
+      if (ksrc)
+        *reinterpret_cast<uint4*>(a.tk + ((b * a.H + h) * a.t_rows + kpos + r) * kHeadDim + c * 8) =
+            *reinterpret_cast<const uint4*>(ksrc + row * a.tkj + c * 8);
+    }
+    uint32_t* d = rows32 + r * 65 + c * 4;
+    d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+  }
+  __syncthreads();
+  // chunk ch = 2 g + s of dim rows 2 p and 2 p + 1: the keys 16 g + 4 s + 0..3 and 16 g + 8 + 4 s + 0..3
+  uint16_t* out = a.vt + b * a.svb + h * a.svh + tile * kBK;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    const int ch = tid & 7, p = (tid >> 3) + 32 * u;
+    uint32_t x[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[e] = rows32[((ch >> 1) * 16 + (e >> 2) * 8 + (ch & 1) * 4 + (e & 3)) * 65 + p];
+    uint4 lo, hi;
+    lo.x = __builtin_amdgcn_perm(x[1], x[0], 0x05040100u); hi.x = __builtin_amdgcn_perm(x[1], x[0], 0x07060302u);
+    lo.y = __builtin_amdgcn_perm(x[3], x[2], 0x05040100u); hi.y = __builtin_amdgcn_perm(x[3], x[2], 0x07060302u);
+    lo.z = __builtin_amdgcn_perm(x[5], x[4], 0x05040100u); hi.z = __builtin_amdgcn_perm(x[5], x[4], 0x07060302u);
+    lo.w = __builtin_amdgcn_perm(x[7], x[6], 0x05040100u); hi.w = __builtin_amdgcn_perm(x[7], x[6], 0x07060302u);
+    *reinterpret_cast<uint4*>(out + (2 * p) * a.svd + ch * 8) = lo;
+    *reinterpret_cast<uint4*>(out + (2 * p + 1) * a.svd + ch * 8) = hi;
+  }
+}
+
+// Launches the attention kernel over args whose pointers, strides, segments and groups are set.
+int launch_attention(AttnArgs& a, int64_t B, float scale, hipStream_t st) {
+  int64_t qblocks = 0;
+  for (int g = 0; g < a.ngroups; g++) {
+    a.group[g].qb0 = (int)qblocks;
+    qblocks += ((int64_t)a.group[g].q_n + kBQ - 1) / kBQ;
+  }
+  const int64_t grid = B * a.H * qblocks;
+  HN_REQUIRE(grid <= 0x7fffffff, "hn_attention: problem too large");
+  if (grid == 0) return HN_OK;
+  a.scale_log2 = scale * 1.4426950408889634f;
+  a.qblocks = (int)qblocks;
+  hipLaunchKernelGGL(attention_kernel, dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, st, a);
+  return HN_LAUNCH_CHECK("attention_kernel");
+}
+
+int64_t tiles_of(int64_t n) { return (n + kBK - 1) / kBK; }
+
+// The workspace of hn_segment_attention: V^T [B, H, 128, positions], packed text keys [B, H, t_rows, 128], the
+// owner of each query row; each from a 256-byte boundary.
+struct SegmentLayout {
+  int64_t positions, t_rows, vt, tk, owner, bytes;
+};
+SegmentLayout segment_layout(const int64_t* parts, int n_parts, const int64_t* groups, int n_groups, int64_t B,
+                             int64_t H, int64_t Lq) {
+  SegmentLayout l{};
+  for (int g = 0; g < n_groups; g++) l.t_rows += tiles_of(groups[4 * g + 3]) * kBK;
+  l.positions = l.t_rows;
+  for (int p = 0; p < n_parts; p++) l.positions += tiles_of(parts[9 * p + 8]) * kBK;
+  auto align = [](int64_t x) { return (x + 255) / 256 * 256; };
+  l.tk = align(B * H * kHeadDim * l.positions * 2);
+  l.owner = l.tk + align(B * H * kHeadDim * l.t_rows * 2);
+  l.bytes = l.owner + (n_groups ? align(Lq * 4) : 0);
+  return l;
 }
 
 }  // namespace
@@ -307,18 +516,112 @@ extern "C" int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi
              "hn_attention: key stride %lld / V^T row stride %lld out of range (tile offsets are 32-bit)",
              (long long)skj, (long long)svd);
   HN_REQUIRE(scale > 0.0f && scale < 1e30f, "hn_attention: bad scale");
+  HN_REQUIRE(Lq <= 0x7fffffff - kBQ && Lk <= ((int64_t)1 << 36) && H <= 0x7fffffff, "hn_attention: problem too large");
   if (B == 0 || Lq == 0) return HN_OK;
-  const int64_t qblocks = (Lq + kBQ - 1) / kBQ;
-  const int64_t grid = B * H * qblocks;
-  HN_REQUIRE(grid <= 0x7fffffff && qblocks <= 0x7fffffff && H <= 0x7fffffff, "hn_attention: problem too large");
   AttnArgs a{};
   a.q = (const uint16_t*)q; a.sqb = sqb; a.sqh = sqh; a.sqi = sqi;
-  a.k = (const uint16_t*)k; a.skb = skb; a.skh = skh; a.skj = skj;
+  a.seg[0] = AttnSeg{(const uint16_t*)k, skb, skh, skj, Lk, 0};
+  a.nseg = 1;
   a.vt = (const uint16_t*)vt; a.svb = svb; a.svh = svh; a.svd = svd;
   a.o = (uint16_t*)out; a.sob = sob; a.soh = soh; a.soi = soi;
-  a.H = (int)H; a.Lq = Lq; a.Lk = Lk;
-  a.scale_log2 = scale * 1.4426950408889634f;
-  a.qblocks = (int)qblocks;
-  hipLaunchKernelGGL(attention_kernel, dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, (hipStream_t)stream, a);
-  return HN_LAUNCH_CHECK("attention_kernel");
+  a.H = (int)H;
+  a.ngroups = 1;
+  a.group[0] = AttnGroup{0, 0, (int)Lq, 0, 0};
+  return launch_attention(a, B, scale, (hipStream_t)stream);
+}
+
+extern "C" int64_t hn_segment_attention_workspace_bytes(const int64_t* parts, int n_parts, const int64_t* groups,
+                                                        int n_groups, int64_t B, int64_t H, int64_t Lq) {
+  using namespace hn;
+  if (!parts || n_parts < 1 || n_parts > 2 || n_groups < 0 || n_groups > kMaxGroups || (n_groups && !groups) || B < 0 ||
+      H <= 0 || Lq < 0)
+    return -1;
+  return segment_layout(parts, n_parts, groups, n_groups, B, H, Lq).bytes;
+}
+
+extern "C" int hn_segment_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const int64_t* parts,
+                                    int n_parts, const int64_t* text, const int64_t* groups, int n_groups,
+                                    const int64_t* rows, int64_t text_off, void* out, int64_t sob, int64_t soh,
+                                    int64_t soi, int64_t B, int64_t H, int64_t Lq, int64_t D, float scale,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace hn;
+  HN_REQUIRE(B >= 0 && H > 0 && H <= 65535 && B * H <= 65535 && Lq >= 0 && Lq <= 0x7fffffff - kBQ,
+             "hn_segment_attention: bad shape B=%lld H=%lld Lq=%lld", (long long)B, (long long)H, (long long)Lq);
+  HN_REQUIRE(D == kHeadDim, "hn_segment_attention: head dim %lld (128 only)", (long long)D);
+  HN_REQUIRE(n_parts >= 1 && n_parts <= 2 && parts, "hn_segment_attention: one or two shared key parts, got %d", n_parts);
+  HN_REQUIRE(n_groups >= 0 && n_groups <= kMaxGroups, "hn_segment_attention: at most %d query groups, got %d", kMaxGroups,
+             n_groups);
+  HN_REQUIRE(n_groups == 0 || (groups && rows && text), "hn_segment_attention: groups without rows or text source");
+  HN_REQUIRE(q && out && workspace, "hn_segment_attention: null pointer");
+  HN_REQUIRE(scale > 0.0f && scale < 1e30f, "hn_segment_attention: bad scale");
+  auto rows16 = [](const int64_t* t) {  // pointer, then batch / head / token strides: 16-byte aligned rows
+    return t[0] != 0 && (t[0] & 15) == 0 && t[1] % 8 == 0 && t[2] % 8 == 0 && t[3] % 8 == 0 && t[3] > 0 && t[3] <= (1 << 23);
+  };
+  int64_t shared = 0;
+  for (int p = 0; p < n_parts; p++) {
+    HN_REQUIRE(rows16(parts + 9 * p) && rows16(parts + 9 * p + 4) && parts[9 * p + 8] >= 0,
+               "hn_segment_attention: key part %d must have 16-byte aligned rows, token strides in (0, 2^23]", p);
+    shared += parts[9 * p + 8];
+  }
+  HN_REQUIRE(((uintptr_t)q & 15) == 0 && sqb % 8 == 0 && sqh % 8 == 0 && sqi % 8 == 0 && ((uintptr_t)out & 7) == 0 &&
+                 sob % 4 == 0 && soh % 4 == 0 && soi % 4 == 0,
+             "hn_segment_attention: q rows must be 16-byte and out rows 8-byte aligned");
+  HN_REQUIRE(n_groups == 0 || (rows16(text) && rows16(text + 4)), "hn_segment_attention: text rows must be 16-byte aligned");
+  const SegmentLayout l = segment_layout(parts, n_parts, groups, n_groups, B, H, Lq);
+  HN_REQUIRE(l.positions <= (1 << 22), "hn_segment_attention: %lld key positions (at most 2^22)", (long long)l.positions);
+  HN_REQUIRE(workspace_bytes >= l.bytes && ((uintptr_t)workspace & 255) == 0,
+             "hn_segment_attention: workspace of %lld bytes (256-byte aligned), %lld needed", (long long)workspace_bytes,
+             (long long)l.bytes);
+  for (int g = 0; g < n_groups; g++) {
+    const int64_t* w = groups + 4 * g;
+    HN_REQUIRE(w[0] >= 0 && w[1] >= 0 && w[2] >= 0 && w[3] >= 0 && w[0] + w[1] <= 0x7fffffff && w[2] + w[3] <= 0x7fffffff,
+               "hn_segment_attention: bad group %d", g);
+    HN_REQUIRE(w[1] == 0 || shared + w[3] > 0, "hn_segment_attention: no keys for group %d", g);
+  }
+  HN_REQUIRE(n_groups > 0 || Lq == 0 || shared > 0, "hn_segment_attention: no keys");
+  if (B == 0 || Lq == 0) return HN_OK;
+
+  char* ws = (char*)workspace;
+  AttnArgs a{};
+  PackArgs p{};
+  a.q = (const uint16_t*)q; a.sqb = sqb; a.sqh = sqh; a.sqi = sqi;
+  a.vt = (const uint16_t*)ws;
+  a.svd = l.positions; a.svh = kHeadDim * l.positions; a.svb = H * a.svh;
+  a.o = (uint16_t*)out; a.sob = sob; a.soh = soh; a.soi = soi;
+  a.H = (int)H;
+  p.vt = (uint16_t*)ws; p.svb = a.svb; p.svh = a.svh; p.svd = a.svd; p.H = (int)H; p.Lq = Lq;
+  int64_t tile = 0;
+  for (int i = 0; i < n_parts; i++) {
+    const int64_t* w = parts + 9 * i;
+    a.seg[i] = AttnSeg{(const uint16_t*)w[0], w[1], w[2], w[3], w[8], tile * kBK};
+    p.part[i] = PackPart{(const uint16_t*)w[4], w[5], w[6], w[7], w[8], tile};
+    tile += tiles_of(w[8]);
+  }
+  a.nseg = p.nparts = n_parts;
+  p.text_tile0 = tile;
+  a.tvpos = tile * kBK;
+  p.tiles = l.positions / kBK;
+  a.t_rows = p.t_rows = l.t_rows;
+  a.ngroups = 1;
+  a.group[0] = AttnGroup{0, 0, (int)Lq, 0, 0};
+  if (n_groups) {
+    a.tk = p.tk = (uint16_t*)(ws + l.tk);
+    a.owner = p.owner = (int*)(ws + l.owner);
+    a.rows = p.rows = rows;
+    p.text_off = text_off;
+    p.tk_src = (const uint16_t*)text[0]; p.tkb = text[1]; p.tkh = text[2]; p.tkj = text[3];
+    p.tv_src = (const uint16_t*)text[4]; p.tvb = text[5]; p.tvh = text[6]; p.tvj = text[7];
+    a.ngroups = p.ngroups = n_groups;
+    int64_t pos = 0;
+    for (int g = 0; g < n_groups; g++) {
+      const int64_t* w = groups + 4 * g;
+      a.group[g] = p.group[g] = AttnGroup{0, (int)w[0], (int)w[1], (int)w[3], (int)pos};
+      p.t_off[g] = (int)w[2];
+      pos += tiles_of(w[3]) * kBK;
+    }
+  }
+  const dim3 grid((unsigned)(p.tiles + (n_groups ? 1 : 0)), (unsigned)(B * H));
+  hipLaunchKernelGGL(attention_pack_kernel, grid, dim3(kPackThreads), 0, (hipStream_t)stream, p);
+  const int rc = HN_LAUNCH_CHECK("attention_pack_kernel");
+  return rc != HN_OK ? rc : launch_attention(a, B, scale, (hipStream_t)stream);
 }

@@ -39,6 +39,9 @@ SIGNATURES = {
                                  _i, _i64, _p], _i),
     "hn_attention": ([_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64,
                       _i64, _i64, _i64, _i64, _f, _p], _i),
+    "hn_segment_attention_workspace_bytes": ([_p, _i, _p, _i, _i64, _i64, _i64], _i64),
+    "hn_segment_attention": ([_p, _i64, _i64, _i64, _p, _i, _p, _p, _i, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64,
+                              _i64, _f, _p, _i64, _p], _i),
     "hn_adaln": ([_p, _p, _p, _i, _i64, _i64, _i64, _f, _i, _p, _p], _i),
     "hn_adaln_quant": ([_p, _p, _p, _i, _i64, _i64, _i64, _f, _i, _i, _i64, _p, _p, _p], _i),
     "hn_gated_residual": ([_p, _p, _p, _i, _i64, _i64, _i64, _p, _p], _i),
@@ -93,6 +96,11 @@ def stream(t):
 
 def ptr(t):
     return t.data_ptr() if t is not None else None
+
+
+def int64s(values):
+    """A host array of int64 values for an entry point that takes a table."""
+    return (_i64 * len(values))(*values)
 
 
 def dtype_code(t):

@@ -21,6 +21,8 @@ from . import _lib
 
 BACKEND_ENV = "HY_NOMAS_ATTENTION"
 KEY_TILE = 64          # keys per tile of the kernel; V^T rows are padded to a multiple of it
+MAX_GROUPS = 64        # query groups of one hn_segment_attention call
+MAX_POSITIONS = 1 << 22  # its V^T row length
 
 
 def choose_backend(name=None):
@@ -108,9 +110,92 @@ def attention_hip(q, k, vt, lk, out=None, scale=None):
     return out
 
 
+def _operand(t):
+    """Pointer and batch / head / token strides of [B, L, H, D]."""
+    return t.data_ptr(), t.stride(0), t.stride(2), t.stride(1)
+
+
+def _parts_ok(q, parts):
+    """Whether `hn_segment_attention` takes these operands: bf16, head dim 128, one or two (k, v) parts of q's
+    device, batch and heads, k and v of one shape, token strides its 32-bit tile offsets hold."""
+    b, _, h, d = q.shape
+    return (0 < len(parts) <= 2 and b * h <= 65535 and q.numel() > 0
+            and all(_hip_ok(q, k, v) and k.device == v.device == q.device and k.shape == v.shape and k.dim() == 4
+                    and (k.shape[0], k.shape[2]) == (b, h) and 0 < k.stride(1) <= 1 << 23 and 0 < v.stride(1) <= 1 << 23
+                    for k, v in parts)
+            and sum(_tiled(k.shape[1]) for k, _ in parts) <= MAX_POSITIONS)
+
+
+def _tiled(n):
+    return -(-n // KEY_TILE) * KEY_TILE
+
+
+def _attend_parts(q, parts, out=None):
+    """Attention of every query to the keys of all (k, v) `parts`, read where they lie."""
+    q = _rows16(q)
+    parts = [(_rows16(k), _rows16(v)) for k, v in parts]
+    if out is None:
+        out = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16)
+    _segment_call(q, parts, None, [], None, 0, out)
+    return out
+
+
+def _segment_call(q, parts, text, groups, rows, text_off, out):
+    b, lq, h, d = q.shape
+    pt = _lib.int64s([x for k, v in parts for x in (*_operand(k), *_operand(v), k.shape[1])])
+    tx = _lib.int64s([*_operand(text[0]), *_operand(text[1])]) if text is not None else None
+    gr = _lib.int64s([x for g in groups for x in g]) if groups else None
+    nbytes = _lib.lib().hn_segment_attention_workspace_bytes(pt, len(parts), gr, len(groups), b, h, lq)
+    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
+    _lib.call("hn_segment_attention", *_operand(q), pt, len(parts), tx, gr, len(groups), _lib.ptr(rows), text_off,
+              *_operand(out), b, h, lq, d, d ** -0.5, ws.data_ptr(), nbytes, _lib.stream(q))
+
+
+def _groups_ok(q, k, v, hist, plan, out):
+    """Whether a plan's groups go to `hn_segment_attention`: index vectors on q's device, keys for every group, and
+    an output it can write by rows.  Other forms (masks, host indices, other ranks) take one attention call per
+    group, which also refuses what it refuses."""
+    lv, groups = plan.video_tokens, plan.groups
+    if not (k.shape == v.shape == q.shape and isinstance(groups, (list, tuple)) and groups and isinstance(lv, int)
+            and 0 <= lv <= q.shape[1]
+            and all(len(pair) == 2 and all(isinstance(t, torch.Tensor) and t.dim() == 1 and t.dtype == torch.int64
+                                           and t.device == q.device for t in pair) for pair in groups)
+            and out.stride(3) == 1 and out.data_ptr() % 8 == 0 and all(st % 4 == 0 for st in out.stride()[:3])):
+        return False
+    shared = lv + (hist[0].shape[1] if hist is not None else 0)
+    return ((shared > 0 or all(t.numel() for _, t in groups))
+            and _tiled(shared) + KEY_TILE + sum(_tiled(t.numel()) for _, t in groups) <= MAX_POSITIONS)
+
+
+def _attend_groups(q, k, v, hist, plan, out):
+    """Every query group of a plan in one launch: the history and video keys are shared and read where they lie,
+    each group's text keys gathered.  A row that several groups name takes the last one's result."""
+    lv, length = plan.video_tokens, q.shape[1]
+    q, k, v = _rows16(q), _rows16(k), _rows16(v)
+    parts = [(_rows16(hist[0]), _rows16(hist[1]))] if hist is not None and hist[0].shape[1] else []
+    parts.append((k[:, :lv], v[:, :lv]))
+    for first in range(0, len(plan.groups), MAX_GROUPS):
+        chunk = plan.groups[first:first + MAX_GROUPS]
+        idx = torch.cat([t for t, _ in chunk] + [t for _, t in chunk])
+        nq = sum(t.numel() for t, _ in chunk)
+        if nq < idx.numel():
+            idx[nq:] += lv
+        # torch's own indexing of the row numbers: out-of-range rows are refused and negative ones counted from the
+        # end, as indexing q, k and v themselves does
+        rows = torch.arange(length, device=q.device)[idx]
+        groups, at_q, at_t = [], 0, 0
+        for q_idx, text_idx in chunk:
+            groups.append((at_q, q_idx.numel(), at_t, text_idx.numel()))
+            at_q, at_t = at_q + q_idx.numel(), at_t + text_idx.numel()
+        _segment_call(q, parts, (k, v), groups, rows, nq, out)
+    return out
+
+
 def attention(q, k, v, transformer_options=None, *, backend=None):
     """q [B, Lq, H, D], k / v [B, Lk, H, D] -> [B, Lq, H, D] (hy_nomas/model.py:145-150)."""
     if choose_backend(backend) == "hip" and _hip_ok(q, k, v):
+        if k.shape[1] and _parts_ok(q, [(k, v)]):
+            return _attend_parts(q, [(k, v)])
         vt = transpose_values(v.transpose(1, 2))
         return attention_hip(q, k, vt, k.shape[1])
     return sdpa(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)).transpose(1, 2)
@@ -120,6 +205,9 @@ def attention_heads(qh, kh, vh, backend=None):
     """`attention` on head-major operands qh [B, H, Lq, D], kh / vh [B, H, Lk, D] (as the QKV epilogue writes
     them).  Returns [B, Lq, H, D] (a view for SDPA, a contiguous tensor for the HIP kernel)."""
     if choose_backend(backend) == "hip" and _hip_ok(qh, kh, vh):
+        parts = [(kh.transpose(1, 2), vh.transpose(1, 2))]
+        if kh.shape[2] and _parts_ok(qh.transpose(1, 2), parts):
+            return _attend_parts(qh.transpose(1, 2), parts)
         return attention_hip(qh.transpose(1, 2), kh.transpose(1, 2), transpose_values(vh), kh.shape[2])
     return sdpa(qh, kh, vh).transpose(1, 2)
 
@@ -148,16 +236,30 @@ def segment_attention(q, k, v, history, plan, transformer_options=None, *, backe
     tokens first), history (hk, hv) [1 or B, Lh, H, D] or None, plan with `groups` (None: every current token
     queries every key) and `video_tokens`.  Each group's queries attend to the history, every current video key
     and the group's own text keys (indices into the text part)."""
+    return _segment(q, k, v, history, plan, backend)
+
+
+def _segment(q, k, v, history, plan, backend, out=None):
+    """`segment_attention`; with `out`, a plan's groups write their rows there instead of to a new tensor of q's
+    strides."""
     batch = q.shape[0]
     hist = None
     if history is not None:
         hist = tuple(t if t.shape[0] == batch else t.expand(batch, -1, -1, -1) for t in history)
     groups = getattr(plan, "groups", None)
+    hip = choose_backend(backend) == "hip" and _hip_ok(q, k, v)
     if groups is None:
+        parts = [p for p in (hist, (k, v)) if p is not None and p[0].shape[1]]
+        if hip and len(parts) == 2 and _parts_ok(q, parts):
+            return _attend_parts(q, parts)
         return attention(q, *_keys([hist, (k, v)]), backend=backend)
     lv = plan.video_tokens
+    if out is None:
+        out = torch.empty_like(q)
+    if (hip and _groups_ok(q, k, v, hist, plan, out)
+            and _parts_ok(q, [p for p in (hist, (k, v)) if p is not None])):
+        return _attend_groups(q, k, v, hist, plan, out)
     video = (k[:, :lv], v[:, :lv])
-    out = torch.empty_like(q)
     for q_idx, text_idx in groups:
         text = (k[:, lv + text_idx], v[:, lv + text_idx]) if text_idx.numel() else None
         out[:, q_idx] = attention(q[:, q_idx], *_keys([hist, video, text]), backend=backend)

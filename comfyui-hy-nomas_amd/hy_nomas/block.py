@@ -121,7 +121,9 @@ class DoubleStreamBlockInt8:
             out = attn.attention_heads(hm[0], hm[1], hm[2], backend)
         else:
             q, k, v = (t.transpose(1, 2) for t in hm)
-            out = attn.segment_attention(q, k, v, history, plan, backend=backend)
+            # token-major, as the out-projections read it
+            dst = torch.empty(q.shape, device=q.device, dtype=q.dtype)
+            out = attn._segment(q, k, v, history, plan, backend, out=dst)
         del hm
         out = out.reshape(b, out.shape[1], -1)
         img = self.img.post(img, out[:, :lv], gate1, shift2, scale2, gate2)

@@ -187,6 +187,27 @@ int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const voi
                  void* stream);
 
 /*
+ * Attention of one segment over key parts read where they lie.  Replaces segment_attention and its per-group
+ * concatenations (hy_nomas/model.py:199-223).
+ *   parts [n_parts, 9], n_parts 1 or 2, a host table of the keys every query attends to: k pointer and its batch,
+ *   head and token strides, v pointer and its strides, number of keys.  v is as k (no transposed layout).
+ * Without groups (n_groups == 0) every one of the Lq query rows attends to all parts.  With groups (at most 64):
+ *   groups [n_groups, 4], a host table: first query in `rows`, number of queries, first text row (counted from
+ *   rows + text_off), number of text rows; text [8]: k and v pointer and strides of the tensor that the text
+ *   rows index; rows: device int64, every query and text row in range.
+ * A group's queries attend to all parts, then to the group's text rows.  A query row in several groups takes the
+ * last one's result; a row in none is not written.  bf16, D == 128, strides in elements, rows 16-byte aligned
+ * (out 8-byte), token strides of k and v in (0, 2^23]; B * H <= 65535.  The workspace (256-byte aligned) holds V^T
+ * and the gathered text keys: hn_segment_attention_workspace_bytes, which returns -1 for bad counts.
+ */
+int64_t hn_segment_attention_workspace_bytes(const int64_t* parts, int n_parts, const int64_t* groups, int n_groups,
+                                             int64_t B, int64_t H, int64_t Lq);
+int hn_segment_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const int64_t* parts, int n_parts,
+                         const int64_t* text, const int64_t* groups, int n_groups, const int64_t* rows,
+                         int64_t text_off, void* out, int64_t sob, int64_t soh, int64_t soi, int64_t B, int64_t H,
+                         int64_t Lq, int64_t D, float scale, void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * LayerNorm (or RMSNorm) + adaLN modulate.  Replaces fused.adaln / _adaln_kernel (hy_nomas/fused.py:37-62).
  *   x [B, L, D] contiguous (x_dtype bf16 or fp16), shift/scale [B, D] -> y [B, L, D] (same dtype):
  *   y = norm(x) * bf16(1 + scale[b]) + shift[b].

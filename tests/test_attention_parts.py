@@ -1,0 +1,139 @@
+"""Attention over key parts read where they lie (hn_segment_attention, hy_nomas/model.py:199-223): the V^T packing, the
+segments' masked last tiles, the groups' gathered rows, against float32 softmax attention over the joined keys and
+against the one-call-per-group form; and on the CPU, which plans take it and what its entry point refuses."""
+import ctypes
+
+import pytest
+import torch
+
+from conftest import seeded
+from test_attention_gpu import Plan, ref_attention, rel
+
+
+def operands(dev, b, h, lv, lt, lh, seed, head_major=False):
+    g = seeded(seed)
+
+    def make(n, batch=b):
+        if head_major:
+            return torch.randn(batch, h, n, 128, generator=g).to(torch.bfloat16).to(dev).transpose(1, 2)
+        return torch.randn(batch, n, h, 128, generator=g).to(torch.bfloat16).to(dev)
+
+    q, k, v = make(lv + lt), make(lv + lt), make(lv + lt)
+    return q, k, v, (make(lh, 1), make(lh, 1)) if lh else None
+
+
+def split_plan(dev, lv, lt, n):
+    tok, txt = torch.arange(lv, device=dev).tensor_split(n), torch.arange(lt, device=dev).tensor_split(n)
+    return Plan(lv, [(torch.cat([a, lv + t]), t) for a, t in zip(tok, txt)])
+
+
+def per_group(q, k, v, hist, plan):
+    lv, ref = plan.video_tokens, torch.full(q.shape, float("nan"), device=q.device)
+    hk, hv = (t.expand(q.shape[0], -1, -1, -1) for t in hist) if hist else (k[:, :0], v[:, :0])
+    for qi, ti in plan.groups:
+        keys, vals = (torch.cat([x, t[:, :lv], t[:, lv + ti]], dim=1) for x, t in ((hk, k), (hv, v)))
+        ref[:, qi] = ref_attention(q[:, qi], keys, vals)
+    return ref
+
+
+# lengths around the 64-key tile, the 128-query block and the workgroup's 32-query waves; no history, no text keys
+# for a group, more groups than text tokens; token-major and head-major operands; a batch of two over one history
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,h,lv,lt,lh,n,head_major", [
+    (1, 2, 63, 7, 0, 2, False), (1, 3, 64, 64, 64, 1, False), (2, 2, 129, 5, 65, 3, False), (1, 1, 1, 1, 1, 1, True),
+    (2, 3, 300, 130, 191, 4, True), (1, 2, 200, 3, 127, 5, False), (1, 2, 130, 0, 70, 2, False),
+    (1, 1, 150, 70, 33, 70, False)])
+def test_groups_against_float32(dev, b, h, lv, lt, lh, n, head_major):
+    from hy_nomas import attention
+
+    print(f"groups b={b} h={h} lv={lv} lt={lt} lh={lh} n={n} head_major={head_major}", flush=True)
+    q, k, v, hist = operands(dev, b, h, lv, lt, lh, lv + lt + lh, head_major)
+    plan = split_plan(dev, lv, lt, n)
+    got = attention.segment_attention(q, k, v, hist, plan, backend="hip")
+    assert got.stride() == torch.empty_like(q).stride()
+    fro, mx = rel(got, per_group(q, k, v, hist, plan))
+    assert fro < 1e-2 and mx < 3e-2, (fro, mx)  # bf16 operands, probabilities and result, as test_attention_gpu
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lq,lh", [(1, 1), (64, 63), (65, 64), (200, 129)])
+def test_history_without_groups(dev, lq, lh):
+    from hy_nomas import attention
+
+    q, k, v, hist = operands(dev, 1, 2, lq, 0, lh, lq * 3 + lh)
+    got = attention.segment_attention(q, k, v, hist, None, backend="hip")
+    ref = ref_attention(q, torch.cat([hist[0], k], dim=1), torch.cat([hist[1], v], dim=1))
+    fro, mx = rel(got, ref)
+    assert fro < 1e-2 and mx < 3e-2, (fro, mx)
+
+
+@pytest.mark.gpu
+def test_overlapping_negative_and_repeated_rows(dev):
+    """A row in two groups takes the later group's result; negative rows count from the end; a group may name a row
+    twice.  Rows in no group are left alone."""
+    from hy_nomas import attention
+
+    lv, lt = 150, 20
+    q, k, v, hist = operands(dev, 1, 2, lv, lt, 40, 5)
+    at = lambda *x: torch.tensor(x, device=dev)  # noqa: E731
+    plan = Plan(lv, [(torch.arange(0, 100, device=dev), at(0, 1)), (torch.arange(60, 140, device=dev), at(5, -1, 5)),
+                     (at(-1, 3, 3), at(7))])
+    out = torch.zeros_like(q)
+    attention._segment(q, k, v, hist, plan, "hip", out=out)
+    ref = per_group(q, k, v, hist, plan)
+    named = ~ref.isnan().any(-1).any(-1)[0]
+    fro, mx = rel(out[:, named], ref[:, named])
+    assert fro < 1e-2 and mx < 3e-2, (fro, mx)
+    assert (out[:, ~named] == 0).all() and (~named).sum() == lv + lt - 141
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lk", [1, 15, 64, 100, 321])
+def test_packed_values_equal_the_torch_layout(dev, lk):
+    """One part with no groups against the kernel on `transpose_values`: the same products, bit for bit."""
+    from hy_nomas import attention
+
+    q, k, v, _ = operands(dev, 2, 2, lk, 0, 0, lk)
+    got = attention.attention(q, k, v, backend="hip")
+    assert torch.equal(got, attention.attention_hip(q, k, attention.transpose_values(v.transpose(1, 2)), lk))
+
+
+def test_which_plans_take_the_rows():
+    from hy_nomas import attention
+
+    q = torch.empty(1, 12, 1, 128, dtype=torch.bfloat16)
+    good = (torch.arange(10), torch.arange(2))
+
+    def ok(groups, lv=10, hist=None, out=q):
+        return attention._groups_ok(q, q, q, hist, Plan(lv, groups), out)
+
+    assert ok([good]) and ok((good, good)) and ok([good], lv=0)
+    assert not ok([]) and not ok(iter([good])) and not ok([good], lv=13) and not ok([good], lv=-1)
+    for bad in (torch.arange(12) > 3, torch.arange(10, dtype=torch.int32), [0, 1], slice(0, 3), torch.zeros(2, 2).long()):
+        assert not ok([(bad, good[1])]) and not ok([good, (good[0], bad)])
+    assert not ok([(good[0], good[1][:0])], lv=0)  # no keys: the general form refuses it
+    assert ok([(good[0], good[1][:0])], lv=0, hist=(q, q))
+    assert not ok([good], out=torch.empty(1, 12, 128, 1, dtype=torch.bfloat16).transpose(2, 3))
+
+
+def test_argument_validation_without_a_gpu():
+    from hy_nomas import _lib
+
+    lib, p = _lib.lib(), 4096  # never dereferenced: every call below is refused on the host
+
+    def call(parts, groups=(), b=1, h=1, lq=10, d=128, scale=1.0, ws=p, nbytes=1 << 40, rows=p):
+        pt, gr = _lib.int64s(parts), _lib.int64s(groups) if groups else None
+        text = _lib.int64s([p, 0, 128, 128] * 2)
+        return lib.hn_segment_attention(p, 0, 128, 128, pt, len(parts) // 9, text, gr, len(groups) // 4, rows, 0, p, 0, 128,
+                                        128, b, h, lq, d, scale, ws, nbytes, None)
+
+    part = [p, 0, 128, 128, p, 0, 128, 128, 64]
+    for bad in (call(part, d=64), call([]), call(part * 3), call(part[:8] + [0]), call(part, scale=0.0),
+                call([p + 8] + part[1:]), call(part[:3] + [4] + part[4:]), call(part[:7] + [0, 64]),
+                call(part, nbytes=100), call(part, ws=p + 16), call(part, h=70000), call(part, groups=[0, 4, 0, 1], rows=None),
+                call(part[:8] + [0], groups=[0, 4, 0, 0]), call(part, groups=[0, 1, 0, 0] * 65),
+                call(part[:8] + [(1 << 22) + 1])):
+        assert bad != 0 and lib.hn_last_error()
+    assert lib.hn_segment_attention_workspace_bytes(_lib.int64s(part), 1, None, 0, 1, 1, 10) == 128 * 64 * 2
+    assert lib.hn_segment_attention_workspace_bytes(_lib.int64s(part), 3, None, 0, 1, 1, 10) == -1
+    assert ctypes.sizeof(_lib.int64s(part)) == 72
