@@ -89,6 +89,9 @@ struct AttnArgs {
   int H;
   float scale_log2;       // softmax scale times log2(e): the scores are exponentiated base 2
   int qblocks;            // query blocks of one (batch, head)
+  int splits;             // workgroups that share one query block's keys, each a contiguous range of its tiles
+  float4* po;             // splits > 1: unnormalized partial outputs [unit][32 chunks of 4 dims][128 queries]
+  float2* pml;            // and their reference max and sum [unit][128 queries], unit = workgroup
   int ngroups;
   AttnGroup group[kMaxGroups];
 };
@@ -102,13 +105,16 @@ __device__ __forceinline__ float max_xor32(float x) {
   return __builtin_fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
 }
 
+template <bool SPLIT>
 __global__ __launch_bounds__(kAttnWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void attention_kernel(const AttnArgs a) {
   __shared__ __align__(16) char smem[2 * kAttnStage];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h2 = lane >> 5, l32 = lane & 31;
-  const int bh = blockIdx.x / a.qblocks, qb = blockIdx.x % a.qblocks;
+  // the workgroups of one (batch, head) and key range run side by side, so their tiles are read once from HBM
+  const int range = blockIdx.x / a.qblocks, qb = blockIdx.x % a.qblocks;
+  const int bh = SPLIT ? range / a.splits : range, split = SPLIT ? range % a.splits : 0;
   const int64_t b = bh / a.H, hh = bh % a.H;
   int gi = 0;
   while (gi + 1 < a.ngroups && qb >= a.group[gi + 1].qb0) gi++;
@@ -210,6 +216,18 @@ void attention_kernel(const AttnArgs a) {
 
   int nt = (t_n + kBK - 1) / kBK;  // tiles of all segments
   for (int i = 0; i < a.nseg; i++) nt += (int)((a.seg[i].len + kBK - 1) / kBK);
+  next_segment();
+  if constexpr (SPLIT) {  // this workgroup's tiles [skip, skip + nt)
+    int skip = (int)((int64_t)nt * split / a.splits);
+    nt = (int)((int64_t)nt * (split + 1) / a.splits) - skip;
+    for (int64_t here; (here = (left + kBK - 1) / kBK) <= skip;) {
+      skip -= (int)here;
+      next_segment();
+    }
+    kcur += (int64_t)skip * kBK * kstride;
+    vcur += (int64_t)skip * kBK * 2;
+    left -= (int64_t)skip * kBK;
+  }
   int keys = 0, keys_next = 0;     // keys of the current and of the loading tile
   // tile t in stage buffer BUF (a constant, so the buffer offset rides in the LDS reads' immediate field
   // and the lane's fragment offsets stay fixed across the loop)
@@ -323,7 +341,6 @@ void attention_kernel(const AttnArgs a) {
         }
       }
   };
-  next_segment();
   keys_next = issue_tile(0);
   for (int t = 0; t < nt; t += 2) {
     tile(t, std::integral_constant<int, 0>());
@@ -333,6 +350,17 @@ void attention_kernel(const AttnArgs a) {
   for (int i = 0; i < 32; i++) lsum += pv[i];
   // normalize and store: lane holds query l32, dims 32 db + 8 rr + 4 h2 + 0..3 in registers 4 rr .. 4 rr + 3
   const float ltot = lsum + __shfl_xor(lsum, 32);
+  if constexpr (SPLIT) {  // fp32 partials, 16 bytes per lane with the 32 queries side by side
+    float4* po = a.po + (int64_t)blockIdx.x * 32 * kBQ + wave * 32 + l32;
+#pragma unroll
+    for (int db = 0; db < 4; db++)
+#pragma unroll
+      for (int rr = 0; rr < 4; rr++)
+        po[(8 * db + 2 * rr + h2) * kBQ] =
+            make_float4(oacc[db][4 * rr], oacc[db][4 * rr + 1], oacc[db][4 * rr + 2], oacc[db][4 * rr + 3]);
+    if (h2 == 0) a.pml[(int64_t)blockIdx.x * kBQ + wave * 32 + l32] = make_float2(m, ltot);
+    return;
+  }
   const float inv = 1.0f / ltot;
   if (q0 + l32 < q_n && (a.owner == nullptr || a.owner[qrow] == gi)) {
     uint16_t* orow = a.o + b * a.sob + hh * a.soh + qrow * a.soi;
@@ -346,6 +374,50 @@ void attention_kernel(const AttnArgs a) {
         *reinterpret_cast<uint2*>(orow + d) = w;
       }
   }
+}
+
+// The result of queries whose keys were split: out = sum_s w_s O_s / sum_s w_s l_s with w_s = exp2(m_s - max m).
+// A workgroup takes 32 queries of one query block, a thread 16 dims of one query; bound by reading the partials
+// (64 KB per 128 queries and split).
+constexpr int kCombineThreads = 256;
+
+__global__ __launch_bounds__(kCombineThreads) void attention_combine_kernel(const AttnArgs a) {
+  const int ql = (blockIdx.x % 4) * 32 + (threadIdx.x & 31), part = threadIdx.x >> 5;
+  const int unit = blockIdx.x / 4;
+  const int bh = unit / a.qblocks, qb = unit % a.qblocks;
+  int gi = 0;
+  while (gi + 1 < a.ngroups && qb >= a.group[gi + 1].qb0) gi++;
+  const int qi = (qb - a.group[gi].qb0) * kBQ + ql;
+  if (qi >= a.group[gi].q_n) return;
+  const int64_t qrow = a.rows ? a.rows[a.group[gi].q_off + qi] : qi;
+  if (a.owner != nullptr && a.owner[qrow] != gi) return;
+  const int64_t first = (int64_t)bh * a.splits * a.qblocks + qb;  // the unit's workgroup of split s: first + s qblocks
+  float mmax = -__builtin_inff();
+  for (int s = 0; s < a.splits; s++) mmax = __builtin_fmaxf(mmax, a.pml[(first + (int64_t)s * a.qblocks) * kBQ + ql].x);
+  float o[16], l = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; i++) o[i] = 0.0f;
+  for (int s = 0; s < a.splits; s++) {
+    const int64_t wg = first + (int64_t)s * a.qblocks;
+    const float2 ml = a.pml[wg * kBQ + ql];
+    const float w = __builtin_amdgcn_exp2f(ml.x - mmax);
+    l = __builtin_fmaf(w, ml.y, l);
+    const float4* po = a.po + (wg * 32 + part * 4) * kBQ + ql;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const float4 v = po[c * kBQ];
+      o[4 * c] = __builtin_fmaf(w, v.x, o[4 * c]);
+      o[4 * c + 1] = __builtin_fmaf(w, v.y, o[4 * c + 1]);
+      o[4 * c + 2] = __builtin_fmaf(w, v.z, o[4 * c + 2]);
+      o[4 * c + 3] = __builtin_fmaf(w, v.w, o[4 * c + 3]);
+    }
+  }
+  const float inv = 1.0f / l;
+  uint16_t* orow = a.o + (bh / a.H) * a.sob + (bh % a.H) * a.soh + qrow * a.soi + part * 16;
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+    *reinterpret_cast<uint2*>(orow + 4 * c) = make_uint2(bf16x2_finite(o[4 * c] * inv, o[4 * c + 1] * inv),
+                                                         bf16x2_finite(o[4 * c + 2] * inv, o[4 * c + 3] * inv));
 }
 
 // V^T of every key segment, and the packed text keys, for attention_kernel.
@@ -455,49 +527,102 @@ __global__ __launch_bounds__(kPackThreads) void attention_pack_kernel(const Pack
   }
 }
 
-// Launches the attention kernel over args whose pointers, strides, segments and groups are set.
-int launch_attention(AttnArgs& a, int64_t B, float scale, hipStream_t st) {
+int64_t tiles_of(int64_t n) { return (n + kBK - 1) / kBK; }
+
+// How many workgroups share one query block's keys, from the number of query blocks (units) and their key tiles.
+// Times are in tiles of a compute unit that holds two workgroups: a round of workgroups takes its tiles plus about
+// four for its start and end, a last round of at most one workgroup per unit 0.7 of that (its waves have the SIMD
+// to themselves), a combine pass its launch and 128 KB of traffic per workgroup.  Ranges stay at four tiles or
+// more, workgroups at four rounds (the partials' memory), and a split has to promise a twentieth.  Measured whole
+// calls, one range against the chosen number: 16 units x 290 tiles 316 -> 61 us, 40 x 73 89 -> 40, 144 x 49 69 -> 58,
+// 216 x 129 191 -> 148, 336 x 182 330 -> 281, 592 x 213 618 -> 527; from about two rounds of units up the best
+// number gains under 2 % and one range stays.  The choice lies within 5 % of the best of 1 to 32 throughout.
+int choose_splits(int64_t units, int64_t tiles) {
+  const int64_t cus = cu_count(), slots = 2 * cus;
+  auto cost = [&](int64_t s) {
+    const int64_t full = units * s / slots, rem = units * s % slots;
+    const double rounds = full + (rem == 0 ? 0.0 : rem <= cus ? 0.7 : 1.0);
+    return rounds * ((tiles + s - 1) / s + 4) + (s > 1 ? 2.0 + 0.016 * units * s : 0.0);
+  };
+  int best = 1;
+  double least = 0.95 * cost(1);
+  for (int64_t s = 2; s <= 64 && s * 4 <= tiles && units * s <= 4 * slots; s++)
+    if (cost(s) < least) {
+      best = (int)s;
+      least = cost(s);
+    }
+  return best;
+}
+
+// Bytes of the partials of `units` query blocks in `splits` ranges: outputs, then maxima and sums.
+int64_t partial_bytes(int64_t units, int splits) {
+  return splits > 1 ? units * splits * kBQ * (kHeadDim * 4 + 8) : 0;
+}
+
+// Launches the attention kernel over args whose pointers, strides, segments and groups are set; `partials` is
+// where the partials of `splits` > 1 go.
+int launch_attention(AttnArgs& a, int64_t B, float scale, int splits, char* partials, hipStream_t st) {
   int64_t qblocks = 0;
   for (int g = 0; g < a.ngroups; g++) {
     a.group[g].qb0 = (int)qblocks;
     qblocks += ((int64_t)a.group[g].q_n + kBQ - 1) / kBQ;
   }
-  const int64_t grid = B * a.H * qblocks;
-  HN_REQUIRE(grid <= 0x7fffffff, "hn_attention: problem too large");
-  if (grid == 0) return HN_OK;
+  const int64_t units = B * a.H * qblocks;
+  HN_REQUIRE(units * splits <= 0x7fffffff, "hn_attention: problem too large");
+  if (units == 0) return HN_OK;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.qblocks = (int)qblocks;
-  hipLaunchKernelGGL(attention_kernel, dim3((unsigned)grid), dim3(kAttnWaves * 64), 0, st, a);
-  return HN_LAUNCH_CHECK("attention_kernel");
+  a.splits = splits;
+  const dim3 grid((unsigned)(units * splits)), block(kAttnWaves * 64);
+  if (splits == 1) {
+    hipLaunchKernelGGL(attention_kernel<false>, grid, block, 0, st, a);
+    return HN_LAUNCH_CHECK("attention_kernel");
+  }
+  a.po = (float4*)partials;
+  a.pml = (float2*)(partials + units * splits * kBQ * kHeadDim * 4);
+  hipLaunchKernelGGL(attention_kernel<true>, grid, block, 0, st, a);
+  const int rc = HN_LAUNCH_CHECK("attention_kernel");
+  if (rc != HN_OK) return rc;
+  hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)(units * 4)), dim3(kCombineThreads), 0, st, a);
+  return HN_LAUNCH_CHECK("attention_combine_kernel");
 }
 
-int64_t tiles_of(int64_t n) { return (n + kBK - 1) / kBK; }
-
 // The workspace of hn_segment_attention: V^T [B, H, 128, positions], packed text keys [B, H, t_rows, 128], the
-// owner of each query row; each from a 256-byte boundary.
+// owner of each query row, the partials of split keys; each from a 256-byte boundary.
 struct SegmentLayout {
-  int64_t positions, t_rows, vt, tk, owner, bytes;
+  int64_t positions, t_rows, tk, owner, partials, bytes;
+  int splits;
 };
 SegmentLayout segment_layout(const int64_t* parts, int n_parts, const int64_t* groups, int n_groups, int64_t B,
                              int64_t H, int64_t Lq) {
   SegmentLayout l{};
-  for (int g = 0; g < n_groups; g++) l.t_rows += tiles_of(groups[4 * g + 3]) * kBK;
-  l.positions = l.t_rows;
-  for (int p = 0; p < n_parts; p++) l.positions += tiles_of(parts[9 * p + 8]) * kBK;
+  int64_t qblocks = 0, tiles = 0, fewest = -1;  // of all groups; of the shared parts; text tiles of the shortest group
+  for (int g = 0; g < n_groups; g++) {
+    const int64_t q_n = groups[4 * g + 1], t = tiles_of(groups[4 * g + 3]);
+    l.t_rows += t * kBK;
+    qblocks += (q_n + kBQ - 1) / kBQ;
+    if (q_n > 0 && (fewest < 0 || t < fewest)) fewest = t;
+  }
+  if (n_groups == 0) qblocks = (Lq + kBQ - 1) / kBQ;
+  for (int p = 0; p < n_parts; p++) tiles += tiles_of(parts[9 * p + 8]);
+  l.positions = l.t_rows + tiles * kBK;
+  const int64_t units = B * H * qblocks;
+  l.splits = choose_splits(units, tiles + (fewest > 0 ? fewest : 0));  // every group has a tile for every range
   auto align = [](int64_t x) { return (x + 255) / 256 * 256; };
   l.tk = align(B * H * kHeadDim * l.positions * 2);
   l.owner = l.tk + align(B * H * kHeadDim * l.t_rows * 2);
-  l.bytes = l.owner + (n_groups ? align(Lq * 4) : 0);
+  l.partials = l.owner + (n_groups ? align(Lq * 4) : 0);
+  l.bytes = l.partials + partial_bytes(units, l.splits);
   return l;
 }
 
 }  // namespace
 }  // namespace hn
 
-extern "C" int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb,
+static int attention_impl(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb,
                             int64_t skh, int64_t skj, const void* vt, int64_t svb, int64_t svh, int64_t svd,
                             void* out, int64_t sob, int64_t soh, int64_t soi, int64_t B, int64_t H, int64_t Lq,
-                            int64_t Lk, int64_t D, float scale, void* stream) {
+                            int64_t Lk, int64_t D, float scale, void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace hn;
   HN_REQUIRE(B >= 0 && H > 0 && Lq >= 0 && Lk > 0, "hn_attention: bad shape B=%lld H=%lld Lq=%lld Lk=%lld",
              (long long)B, (long long)H, (long long)Lq, (long long)Lk);
@@ -527,7 +652,36 @@ extern "C" int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi
   a.H = (int)H;
   a.ngroups = 1;
   a.group[0] = AttnGroup{0, 0, (int)Lq, 0, 0};
-  return launch_attention(a, B, scale, (hipStream_t)stream);
+  const int64_t units = B * H * ((Lq + kBQ - 1) / kBQ);
+  const int splits = workspace ? choose_splits(units, tiles_of(Lk)) : 1;
+  HN_REQUIRE(workspace_bytes >= partial_bytes(units, splits) && ((uintptr_t)workspace & 15) == 0,
+             "hn_attention_ws: workspace of %lld bytes (16-byte aligned), %lld needed", (long long)workspace_bytes,
+             (long long)partial_bytes(units, splits));
+  return launch_attention(a, B, scale, splits, (char*)workspace, (hipStream_t)stream);
+}
+
+extern "C" int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb,
+                            int64_t skh, int64_t skj, const void* vt, int64_t svb, int64_t svh, int64_t svd,
+                            void* out, int64_t sob, int64_t soh, int64_t soi, int64_t B, int64_t H, int64_t Lq,
+                            int64_t Lk, int64_t D, float scale, void* stream) {
+  return attention_impl(q, sqb, sqh, sqi, k, skb, skh, skj, vt, svb, svh, svd, out, sob, soh, soi, B, H, Lq, Lk, D, scale,
+                        nullptr, 0, stream);
+}
+
+extern "C" int64_t hn_attention_workspace_bytes(int64_t B, int64_t H, int64_t Lq, int64_t Lk) {
+  using namespace hn;
+  if (B < 0 || H <= 0 || Lq < 0 || Lk <= 0) return -1;
+  const int64_t units = B * H * ((Lq + kBQ - 1) / kBQ);
+  return partial_bytes(units, choose_splits(units, tiles_of(Lk)));
+}
+
+extern "C" int hn_attention_ws(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb,
+                               int64_t skh, int64_t skj, const void* vt, int64_t svb, int64_t svh, int64_t svd,
+                               void* out, int64_t sob, int64_t soh, int64_t soi, int64_t B, int64_t H, int64_t Lq,
+                               int64_t Lk, int64_t D, float scale, void* workspace, int64_t workspace_bytes,
+                               void* stream) {
+  return attention_impl(q, sqb, sqh, sqi, k, skb, skh, skj, vt, svb, svh, svd, out, sob, soh, soi, B, H, Lq, Lk, D, scale,
+                        workspace, workspace_bytes, stream);
 }
 
 extern "C" int64_t hn_segment_attention_workspace_bytes(const int64_t* parts, int n_parts, const int64_t* groups,
@@ -623,5 +777,5 @@ extern "C" int hn_segment_attention(const void* q, int64_t sqb, int64_t sqh, int
   const dim3 grid((unsigned)(p.tiles + (n_groups ? 1 : 0)), (unsigned)(B * H));
   hipLaunchKernelGGL(attention_pack_kernel, grid, dim3(kPackThreads), 0, (hipStream_t)stream, p);
   const int rc = HN_LAUNCH_CHECK("attention_pack_kernel");
-  return rc != HN_OK ? rc : launch_attention(a, B, scale, (hipStream_t)stream);
+  return rc != HN_OK ? rc : launch_attention(a, B, scale, l.splits, ws + l.partials, (hipStream_t)stream);
 }

@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "hn_common.h"
 
 namespace hn {
@@ -19,6 +21,20 @@ int hip_status(hipError_t e, const char* what) {
   if (e == hipSuccess) return HN_OK;
   set_error("%s: %s", what, hipGetErrorString(e));
   return HN_ERR_HIP;
+}
+
+// Compute units of the current device.
+// The per-device cache may be filled by several host threads at once; they store the same value.
+int cu_count() {
+  static std::atomic<int> cached[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cached[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
 }
 
 }  // namespace hn

@@ -425,6 +425,7 @@ __device__ __forceinline__ uint32_t pack2_out(float a, float b) {
 namespace hn {
 void set_error(const char* fmt, ...);
 int hip_status(hipError_t e, const char* what);
+int cu_count();  // compute units of the current device
 
 // The one-call linear (linear.hip): workspace size, argument checks, and quantize-then-GEMM into a
 // workspace that holds the activation codes and scales.

@@ -39,6 +39,9 @@ SIGNATURES = {
                                  _i, _i64, _p], _i),
     "hn_attention": ([_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64,
                       _i64, _i64, _i64, _i64, _f, _p], _i),
+    "hn_attention_workspace_bytes": ([_i64, _i64, _i64, _i64], _i64),
+    "hn_attention_ws": ([_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _i64,
+                         _i64, _i64, _i64, _i64, _f, _p, _i64, _p], _i),
     "hn_segment_attention_workspace_bytes": ([_p, _i, _p, _i, _i64, _i64, _i64], _i64),
     "hn_segment_attention": ([_p, _i64, _i64, _i64, _p, _i, _p, _p, _i, _p, _i64, _p, _i64, _i64, _i64, _i64, _i64, _i64,
                               _i64, _f, _p, _i64, _p], _i),

@@ -104,9 +104,12 @@ def attention_hip(q, k, vt, lk, out=None, scale=None):
     if lk == 0:
         raise RuntimeError("attention: no keys")
     scale = d ** -0.5 if scale is None else scale
-    _lib.call("hn_attention", q.data_ptr(), q.stride(0), q.stride(2), q.stride(1), k.data_ptr(), k.stride(0), k.stride(2),
+    nbytes = _lib.lib().hn_attention_workspace_bytes(b, h, lq, lk)
+    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8) if nbytes > 0 else None
+    _lib.call("hn_attention_ws", q.data_ptr(), q.stride(0), q.stride(2), q.stride(1), k.data_ptr(), k.stride(0), k.stride(2),
               k.stride(1), vt.data_ptr(), vt.stride(0), vt.stride(1), vt.stride(2), out.data_ptr(), out.stride(0),
-              out.stride(2), out.stride(1), b, h, lq, lk, d, float(scale), _lib.stream(q))
+              out.stride(2), out.stride(1), b, h, lq, lk, d, float(scale), _lib.ptr(ws), max(nbytes, 0),
+              _lib.stream(q))
     return out
 
 

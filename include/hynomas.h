@@ -187,6 +187,17 @@ int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const voi
                  void* stream);
 
 /*
+ * hn_attention with a workspace (16-byte aligned, hn_attention_workspace_bytes, which may be 0), in which several
+ * workgroups can share a query block's keys where the queries alone would leave the chip idle: each leaves an fp32
+ * partial output with its maximum and sum, and a second pass joins them.
+ */
+int64_t hn_attention_workspace_bytes(int64_t B, int64_t H, int64_t Lq, int64_t Lk);
+int hn_attention_ws(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb, int64_t skh,
+                    int64_t skj, const void* vt, int64_t svb, int64_t svh, int64_t svd, void* out, int64_t sob,
+                    int64_t soh, int64_t soi, int64_t B, int64_t H, int64_t Lq, int64_t Lk, int64_t D, float scale,
+                    void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Attention of one segment over key parts read where they lie.  Replaces segment_attention and its per-group
  * concatenations (hy_nomas/model.py:199-223).
  *   parts [n_parts, 9], n_parts 1 or 2, a host table of the keys every query attends to: k pointer and its batch,
@@ -197,8 +208,8 @@ int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const voi
  *   rows index; rows: device int64, every query and text row in range.
  * A group's queries attend to all parts, then to the group's text rows.  A query row in several groups takes the
  * last one's result; a row in none is not written.  bf16, D == 128, strides in elements, rows 16-byte aligned
- * (out 8-byte), token strides of k and v in (0, 2^23]; B * H <= 65535.  The workspace (256-byte aligned) holds V^T
- * and the gathered text keys: hn_segment_attention_workspace_bytes, which returns -1 for bad counts.
+ * (out 8-byte), token strides of k and v in (0, 2^23]; B * H <= 65535.  The workspace (256-byte aligned) holds V^T,
+ * the gathered text keys and the partials of split keys (hn_attention_ws): hn_segment_attention_workspace_bytes, which returns -1 for bad counts.
  */
 int64_t hn_segment_attention_workspace_bytes(const int64_t* parts, int n_parts, const int64_t* groups, int n_groups,
                                              int64_t B, int64_t H, int64_t Lq);
