@@ -1,6 +1,6 @@
 // Dispatch and C ABI of the block-scaled 8-bit GEMM (hy_nomas/kernels.py:152-170, block_gemm).
 // The kernel template and its design notes are in gemm_kernel.h.
-#include "gemm_kernel.h"
+#include "gemm_launch.h"
 #include "skinny_kernel.h"
 
 namespace hn {
@@ -10,26 +10,6 @@ constexpr int64_t kWholeKInt32Limit = 131072;
 
 // ---------------------------------------------------------------------------------------------
 // configurations
-
-// WPE: waves per SIMD the kernel is compiled for; above WN * WM / 4, several workgroups share a CU and the
-// persistent grid grows to match.
-template <int KIND, int EPI, bool G128, int WN, int WM, int TN, int TM, int OUT_DT, int BK, int NS, bool WBLK = false,
-          int WPE = WN * WM / 4>
-static int launch_cfg(GemmArgs& a, hipStream_t st) {
-  constexpr int BN = WN * TN * 32, BM = WM * TM * 32;
-  const int64_t tm = (a.M + BM - 1) / BM, tn = (a.N + BN - 1) / BN;
-  if (tm * tn > 0x7fffffff) {
-    set_error("hn_block_gemm: problem too large (%lld tiles)", (long long)(tm * tn));
-    return HN_ERR_UNSUPPORTED;
-  }
-  a.tiles_m = (int)tm;
-  a.tiles_n = (int)tn;
-  const int64_t slots = (int64_t)cu_count() * (WPE * 4 / (WN * WM));
-  const int64_t grid = tm * tn < slots ? tm * tn : slots;
-  hipLaunchKernelGGL((block_gemm_kernel<KIND, EPI, G128, WN, WM, TN, TM, OUT_DT, BK, NS, WBLK, WPE>),
-                     dim3((unsigned)grid), dim3(WN * WM * 64), 0, st, a);
-  return HN_LAUNCH_CHECK("block_gemm_kernel");
-}
 
 // The rows of a problem, as two launches: a.M rows from row 0 with the big tile, then the rest with a 128 x 128
 // tile.  Tile rows are independent and every output keeps its fold order, so the results do not depend on
@@ -82,6 +62,10 @@ template <int KIND, int EPI, int OUT_DT>
 static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
   constexpr bool SWIGLU = EPI == HN_EPI_SWIGLU_QUANT;
   constexpr bool SMALL_OK = EPI == HN_EPI_NONE || EPI == HN_EPI_GELU;
+  // epilogues that need a token's 128 channels in one wave: four waves of 128 x 32 where the problem would fill at
+  // most half of the compute units with the big tile (200 x 3072 -> 9216 q/k/v heads 52 -> 25 us g128, 32 -> 19 per
+  // token; -> 12288 GELU + requantization 73 -> 28)
+  constexpr bool WAVE_ROWS = KIND == HN_KIND_INT8 && (EPI == HN_EPI_GELU_QUANT || EPI == kEpiQkvHeads);
   constexpr int ESZ = OUT_DT == HN_DTYPE_F32 ? 4 : 2;
   if (!g128) {
     auto big = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, false, 2, 4, 4, 2, OUT_DT, 128, 2>(x, st); };
@@ -89,6 +73,9 @@ static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
       auto small = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, false, 2, 2, 2, 2, OUT_DT, 128, 2, false, 2>(x, st); };
       return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, small);
     }
+    if constexpr (WAVE_ROWS)
+      if (int64_t rows = 0; choose_tiles(a.M, a.N, 256, 256, cu_count(), &rows) == TileSplit::kSmall)
+        return launch_cfg<KIND, EPI, false, 1, 4, 4, 1, OUT_DT, 128, 2, false, 2>(a, st);
     return big(a);
   }
   if constexpr (KIND == HN_KIND_FP8) {
@@ -112,6 +99,9 @@ static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
       auto small = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, true, 2, 2, 2, 2, OUT_DT, 128, 2, false, 2>(x, st); };
       return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, small);
     }
+    if constexpr (WAVE_ROWS)
+      if (int64_t rows = 0; choose_tiles(a.M, a.N, 256, 256, cu_count(), &rows) == TileSplit::kSmall)
+        return launch_cfg<KIND, EPI, true, 1, 4, 4, 1, OUT_DT, 128, 2, false, 2>(a, st);
     return big(a);
   }
   set_error("hn_block_gemm: swiglu_quant needs per-token scales or fp8 with 128 x 128 block weight scales");
@@ -231,6 +221,14 @@ extern "C" int hn_block_gemm(const void* qa, int64_t lda, const float* sa, int64
     if (!g128) return launch_skinny_mode<0>(a, epilogue, out_dtype, st);
     if (sw_rows == 128) return launch_skinny_mode<2>(a, epilogue, out_dtype, st);
     return launch_skinny_mode<1>(a, epilogue, out_dtype, st);
+  }
+  bool taken = false;
+  if (kind == HN_KIND_INT8 && (!g128 || sw_rows == 1)) {
+    const int rc = launch_ring_int8(a, g128, epilogue, out_dtype, st, &taken);
+    if (taken) return rc;
+  } else if (kind == HN_KIND_FP8 && g128 && sw_rows == 128) {
+    const int rc = launch_ring_fp8(a, epilogue, out_dtype, st, &taken);
+    if (taken) return rc;
   }
   if (kind == HN_KIND_INT8) return launch_kind<HN_KIND_INT8>(a, g128, epilogue, out_dtype, st);
   return launch_kind<HN_KIND_FP8>(a, g128, epilogue, out_dtype, st);

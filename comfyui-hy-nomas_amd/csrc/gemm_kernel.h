@@ -241,7 +241,10 @@ void block_gemm_kernel(const GemmArgs a) {
   constexpr int NW = WN * WM;
   constexpr int BN = WN * TN * 32, BM = WM * TM * 32;
   constexpr int A_BYTES = BN * BK, B_BYTES = BM * BK;
-  constexpr int SC_SLOTS = (BN + BM) / 64;                   // g128: 64-float scale slots per stage
+  // RING: a tile per workgroup and NS > 2 stage buffers, NS - 1 stages of loads in flight (small problems, where
+  // a workgroup has its compute unit's memory pipeline to itself and waits on latency, not on bandwidth)
+  constexpr bool RING = NS > 2;
+  constexpr int SC_SLOTS = BN / 64 + (BM + 63) / 64;         // g128: 64-float scale slots per stage
   constexpr int SC_PER_WAVE = G128 ? (SC_SLOTS + NW - 1) / NW : 0;
   constexpr int SC_BYTES = SC_PER_WAVE * NW * 256;           // g128 scales of one stage
   constexpr int SCR = (NS + 1) * SC_BYTES;                   // the scales' ring, at offset 0
@@ -252,7 +255,7 @@ void block_gemm_kernel(const GemmArgs a) {
   constexpr int SLICES = BK / MF::kSliceK;
   constexpr int STAGES_PER_GROUP = kGroupK / BK;
   static_assert(A_KB * NW * 1024 == A_BYTES && B_KB * NW * 1024 == B_BYTES, "tile rows not divisible among waves");
-  static_assert(NS == 2, "two stage buffers: the next tile's first stage fills buffer 0 during the epilogue");
+  static_assert(NS >= 2 && BN % 64 == 0, "stage buffers and scale slots");
   static_assert(SLICES >= 2 && SLICES % 2 == 0, "fragment sets alternate per slice, starting each stage at set 0");
   static_assert(kGroupK % BK == 0, "stage size");
   static_assert(EPI != HN_EPI_GELU_QUANT || TN * 32 == 128, "gelu_quant needs a 128-channel wave tile");
@@ -262,7 +265,7 @@ void block_gemm_kernel(const GemmArgs a) {
                 "swiglu_quant needs two 128-channel waves per tile row and an even token split");
   // WBLK: one weight-scale row per 128 output channels (the fp8 128 x 128 block layout); a wave's TN * 32
   // channels then lie in one block, so the group fold multiplies by one scale product per token
-  static_assert(!WBLK || (G128 && (TN * 32) % 128 == 0 && BN % 128 == 0), "block weight scales");
+  static_assert(!WBLK || (G128 && 128 % (TN * 32) == 0 && (BN % 128 == 0 || BN == 64)), "block weight scales");
   // RESCALE (fp8 with block weight scales): no separate fp32 running sum.  The matrix core accumulates
   // every group straight into acc, kept in units of the current group's scale product: at each group
   // boundary acc *= ss_g / ss_{g+1} (one VALU op per output, issued block by block between the next
@@ -288,7 +291,7 @@ void block_gemm_kernel(const GemmArgs a) {
   constexpr int EP_OFF = STG_END > RING_END ? STG_END : RING_END;
   constexpr int EP_BYTES = EPI == HN_EPI_ACC32 ? 0 : (2 * BN + BM) * 4;  // sw | bias | sa of the tile
   // (two operand buffers when the next tile's are parked before this tile's epilogue)
-  constexpr int EP_BUFS = STAGED && !G128 && (EPI == HN_EPI_NONE || EPI == HN_EPI_GELU) ? 2 : 1;
+  constexpr int EP_BUFS = !RING && STAGED && !G128 && (EPI == HN_EPI_NONE || EPI == HN_EPI_GELU) ? 2 : 1;
   constexpr int SMEM = EP_OFF + EP_BUFS * EP_BYTES > RING_END ? EP_OFF + EP_BUFS * EP_BYTES : RING_END;
   __shared__ __align__(16) char smem[SMEM];
 
@@ -351,7 +354,7 @@ void block_gemm_kernel(const GemmArgs a) {
     for (int u = 0; u < SC_PER_WAVE; u++) {
       const int q = wave + NW * u;
       if (q < BN / 64) {
-        if constexpr (WBLK) {  // the scale row of the channel's 128-block (n0 is a multiple of 128)
+        if constexpr (WBLK) {  // the scale row of the channel's 128-block (which holds n0 and a 64-channel tile)
           scbase[u] = a.sw + (n0 / 128) * a.ldsw;
           scoff[u] = (uint32_t)(min(q * 64 + lane, nlim) / 128) * (uint32_t)a.ldsw;
         } else {
@@ -407,6 +410,11 @@ void block_gemm_kernel(const GemmArgs a) {
   const int wrow_n = wn * TN * 32 + (lane & 31);  // this lane's A-fragment row within the weight tile
   const int wrow_m = wm * TM * 32 + (lane & 31);  // and B-fragment row within the activation tile
 
+  auto next_buf = [](int buf) __attribute__((always_inline)) {
+    if constexpr (NS == 2) return buf ^ 1;
+    else if constexpr ((NS & (NS - 1)) == 0) return (buf + 1) & (NS - 1);
+    else return buf + 1 < NS ? buf + 1 : 0;
+  };
   // Fragments are read one MFMA slice ahead of the slice being multiplied (two register sets); the
   // stage barrier sits between the last slice's reads and its MFMAs.
   Frag fa[2][TN], fb[2][TM];
@@ -425,8 +433,8 @@ void block_gemm_kernel(const GemmArgs a) {
   // folded during the next stage's first block (and after the tile's last stage).  The activation fragments
   // of every token block and slice are read once per stage and stay in registers; the weight fragments of
   // channel block i + 1 replace those of block i slice by slice during block i's last token block.
-  constexpr bool BMAJ = G128 && !RESCALE && !WBLK && STAGES_PER_GROUP == 1;
-  static_assert(!BMAJ || TM >= 2, "the weight fragments of the next channel block are read during the last token block");
+  // (it needs two token blocks: the next channel block's weight fragments are read during the last one)
+  constexpr bool BMAJ = G128 && !RESCALE && !WBLK && STAGES_PER_GROUP == 1 && TM >= 2;
   Frag fbs[BMAJ ? TM : 1][BMAJ ? SLICES : 1], fas[BMAJ ? SLICES : 1];
 
   // The tile's epilogue operands (per-channel weight scale and bias, per-token activation scale), parked in
@@ -439,7 +447,9 @@ void block_gemm_kernel(const GemmArgs a) {
   // youngest vector-memory ops; the counter retires in issue order) in flight under its first products.
   constexpr int EP_PER = EPI == HN_EPI_ACC32 ? 0 : (BN + NW * 64 - 1) / (NW * 64);
   constexpr int EPM_PER = EPI == HN_EPI_ACC32 || G128 ? 0 : (BM + NW * 64 - 1) / (NW * 64);
-  constexpr bool EARLY_EP = STAGED && !G128 && (EPI == HN_EPI_NONE || EPI == HN_EPI_GELU);
+  // Ring tiles fetch theirs before the first stage and park them after the last, so nothing waits for them.
+  constexpr bool EARLY_EP = !RING && STAGED && !G128 && (EPI == HN_EPI_NONE || EPI == HN_EPI_GELU);
+  constexpr bool EP_BITS = EARLY_EP || RING;  // the bias is held as raw bits until it is parked
   constexpr int NST = TM * 32 / (64 / (TN * 32 * 2 / 16));  // the staged epilogue's stores per full tile
   static_assert(NST < 64, "vmcnt range");
   float ep_sw[EP_PER > 0 ? EP_PER : 1], ep_b[EP_PER > 0 ? EP_PER : 1], ep_sa[EPM_PER > 0 ? EPM_PER : 1];
@@ -452,7 +462,7 @@ void block_gemm_kernel(const GemmArgs a) {
       const int tt = tid + u * NW * 64;
       const int64_t n = tn0 + (tt < nlast ? tt : nlast);
       ep_sw[u] = G128 ? 0.0f : a.sw[n * a.ldsw];
-      if constexpr (EARLY_EP) ep_bb[u] = a.bias ? load_bias_bits(a.bias, a.bias_dtype, n) : 0x80000000u;
+      if constexpr (EP_BITS) ep_bb[u] = a.bias ? load_bias_bits(a.bias, a.bias_dtype, n) : 0x80000000u;
       else ep_b[u] = a.bias ? load_bias(a.bias, a.bias_dtype, n) : -0.0f;
     }
 #pragma unroll
@@ -467,7 +477,7 @@ void block_gemm_kernel(const GemmArgs a) {
 #pragma unroll
       for (int u = 0; u < EP_PER; u++) {
         const int tt = tid + u * NW * 64;
-        const float b = EARLY_EP ? (a.bias ? bias_from_bits(ep_bb[u], a.bias_dtype) : -0.0f) : ep_b[u];
+        const float b = EP_BITS ? (a.bias ? bias_from_bits(ep_bb[u], a.bias_dtype) : -0.0f) : ep_b[u];
         if (tt < BN) { ep[tt] = ep_sw[u]; ep[BN + tt] = b; }
       }
 #pragma unroll
@@ -487,7 +497,21 @@ void block_gemm_kernel(const GemmArgs a) {
     fetch_ep(m0, n0);
     write_ep(0);
   }
-  issue_stage(0, 0);
+  if constexpr (RING) {
+    fetch_ep(m0, n0);
+#pragma unroll
+    for (int st = 0; st < NS; st++)
+      if (st < nk) issue_stage(st, st);
+  } else {
+    issue_stage(0, 0);
+  }
+  // RING: wait until all but the `n` youngest of this wave's stages have landed
+  auto wait_stages = [&](int n) __attribute__((always_inline)) {
+    static_for<NS>([&](auto i_c) __attribute__((always_inline)) {
+      constexpr int I = NS - 1 - decltype(i_c)::value;
+      if (n == I) wait_vmcnt<LOADS * I>();
+    });
+  };
 
   for (;;) {
     // A per-tile copy of the lane id that the compiler cannot see through: the lane-dependent index
@@ -515,17 +539,18 @@ void block_gemm_kernel(const GemmArgs a) {
 #pragma unroll
           for (int r = 0; r < 16; r++) facc[i][j][r] = 0.0f;
     }
-    if constexpr (!EARLY_EP) fetch_ep(m0, n0);
+    if constexpr (!EARLY_EP && !RING) fetch_ep(m0, n0);
     // stage 0 (and the epilogue operands) have landed and every wave's staging and operand reads of the
     // previous epilogue are done, so buffer 1 and the operand area are free.  After a full tile of a plain
     // staged epilogue its NST stores are the youngest vector-memory ops and may still be in flight (the
     // counter retires in issue order); otherwise this also retires the previous tile's stores.
-    if (EARLY_EP && stores_full) wait_vmcnt<NST>();
+    if constexpr (RING) wait_stages(nk < NS ? nk - 1 : NS - 1);
+    else if (EARLY_EP && stores_full) wait_vmcnt<NST>();
     else wait_vmcnt<0>();
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     barrier();
-    if constexpr (!EARLY_EP) write_ep(0);
-    if (1 < nk) issue_stage(1, 1);
+    if constexpr (!EARLY_EP && !RING) write_ep(0);
+    if (!RING && 1 < nk) issue_stage(1, 1);
     if constexpr (BMAJ) {
 #pragma unroll
       for (int j = 0; j < TM; j++)
@@ -568,14 +593,14 @@ void block_gemm_kernel(const GemmArgs a) {
     // One K stage (kt, in buffer `buf`).  The schedule is pinned with scheduling barriers (address
     // arithmetic may still move): each slice issues the next slice's fragment reads right after its
     // first products, so they land while the matrix core works.  The last slice holds the stage
-    // barrier; after it the next stage's first fragments are read and the direct loads of stage kt + 2
+    // barrier; after it the next stage's first fragments are read and the direct loads of stage kt + NS
     // are interleaved with the slice's remaining products, so the matrix core is fed while the loads
-    // queue.  MODE 0: barrier and loads; 1: barrier, no loads (stage kt + 2 does not exist); 2: the
+    // queue.  MODE 0: barrier and loads; 1: barrier, no loads (stage kt + NS does not exist); 2: the
     // tile's last stage (neither).
     // Weight rows multiplied before the barrier.  Per-token tiles issue all of the last slice's products
     // after it (1.7 % faster over the DiT stack); the g128 and block-scale tiles keep one row before it
     // (none there is 0.5 % and 3 % slower, two 0.4 % and 2.5 % slower).
-    constexpr int PRE = G128 ? 1 : 0;
+    constexpr int PRE = G128 && TN > 1 ? 1 : 0;
     // the g128 fold (not the rescaled running sum) with one group per stage: every stage starts its partials
     // in its first products, so the fold leaves them as they are
     constexpr bool FRESH = G128 && !RESCALE && STAGES_PER_GROUP == 1;
@@ -585,6 +610,7 @@ void block_gemm_kernel(const GemmArgs a) {
     auto stage_body = [&](int kt, int buf, auto mode_c) __attribute__((always_inline)) {
       constexpr int MODE = decltype(mode_c)::value;
       const char* stage = smem + SCR + buf * STAGE;
+      const char* next = smem + SCR + next_buf(buf) * STAGE;
       // RESCALE: the factor from the previous group's scale product (carried from the previous stage) to this
       // one's (1 at the tile's first stage).
       float rs[TM];
@@ -623,14 +649,15 @@ void block_gemm_kernel(const GemmArgs a) {
           mfma_rows(cur, 0, PRE, nullptr, fresh);
           // (the waits and the barrier are scalar instructions: nothing may cross them)
           __builtin_amdgcn_sched_barrier(0);
-          // stage kt + 1 (the only loads in flight) has landed for this wave and its reads of stage kt
-          // are complete; the barrier publishes both facts, then stage kt + 2 may refill `buf`
-          wait_vmcnt<0>();
+          // stage kt + 1 (the oldest loads in flight) has landed for this wave and its reads of stage kt
+          // are complete; the barrier publishes both facts, then stage kt + NS may refill `buf`
+          if constexpr (MODE == 0 || !RING) wait_vmcnt<LOADS*(NS - 2)>();
+          else wait_stages(nk - 2 - kt);
           __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
           barrier();
           __builtin_amdgcn_sched_barrier(0);
-          read_frags(cur ^ 1, smem + SCR + (buf ^ 1) * STAGE, 0);
-          if constexpr (MODE == 0) issue_stage(kt + 2, buf);
+          read_frags(cur ^ 1, next, 0);
+          if constexpr (MODE == 0) issue_stage(kt + NS, buf);
           mfma_rows(cur, PRE, TN, nullptr, fresh);
           // reads first, then products and loads alternating
           __builtin_amdgcn_sched_group_barrier(0x100, TN + TM, 0);
@@ -733,11 +760,11 @@ void block_gemm_kernel(const GemmArgs a) {
     // its reads before its share of the fold: the group's scales after the first product, the next channel
     // block's weight fragments (slice by slice, as the last token block releases them).  The last channel
     // block follows the stage barrier, reads the next stage's activation fragments as its products release
-    // them, and spreads the direct loads of stage kt + 2 over its products.
+    // them, and spreads the direct loads of stage kt + NS over its products.
     auto bm_stage = [&](int kt, int buf, auto mode_c) __attribute__((always_inline)) {
       constexpr int MODE = decltype(mode_c)::value;
       const char* stage = smem + SCR + buf * STAGE;
-      const char* next = smem + SCR + (buf ^ 1) * STAGE;
+      const char* next = smem + SCR + next_buf(buf) * STAGE;
       // the previous group's last block is folded during this stage's first block, with that group's scales
       const float p_sa = c_sa[TM - 1], p_sw = c_sw[TN - 1];
       static_assert(NB % 2 == 0, "blocks alternate between the two partial sets, block 0 in set 0");
@@ -746,9 +773,10 @@ void block_gemm_kernel(const GemmArgs a) {
         constexpr int pb = (b + NB - 1) % NB, pi = pb / TM, pj = pb % TM;  // the block folded meanwhile
         if constexpr (b == LAST && MODE != 2) {
           // every wave's reads of this stage are done and stage kt + 1 has landed: the barrier publishes
-          // both, then the next stage's fragments are read and stage kt + 2 refills `buf`
+          // both, then the next stage's fragments are read and stage kt + NS refills `buf`
           __builtin_amdgcn_sched_barrier(0);
-          wait_vmcnt<0>();
+          if constexpr (MODE == 0 || !RING) wait_vmcnt<LOADS*(NS - 2)>();
+          else wait_stages(nk - 2 - kt);
           __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
           barrier();
           __builtin_amdgcn_sched_barrier(0);
@@ -768,7 +796,7 @@ void block_gemm_kernel(const GemmArgs a) {
             if constexpr (MODE == 0) {
               constexpr int slot = j * SLICES + s, SLOTS = TM * SLICES;
 #pragma unroll
-              for (int q = slot * LOADS / SLOTS; q < (slot + 1) * LOADS / SLOTS; q++) issue_load(kt + 2, buf, q);
+              for (int q = slot * LOADS / SLOTS; q < (slot + 1) * LOADS / SLOTS; q++) issue_load(kt + NS, buf, q);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -780,8 +808,19 @@ void block_gemm_kernel(const GemmArgs a) {
         });
       });
     };
+    // stages kt = 0 .. nk - 1, each in the buffer after the last one's: MODE 0 while stage kt + NS exists, then
+    // MODE 1 and, for the last stage, MODE 2
     int kt = 0;
-    if constexpr (BMAJ) {
+    if constexpr (RING) {
+      int buf = 0;
+      auto walk = [&](auto&& stage_fn) __attribute__((always_inline)) {
+        for (; kt + NS < nk; kt++, buf = next_buf(buf)) stage_fn(kt, buf, std::integral_constant<int, 0>());
+        for (; kt + 1 < nk; kt++, buf = next_buf(buf)) stage_fn(kt, buf, std::integral_constant<int, 1>());
+        stage_fn(kt, buf, std::integral_constant<int, 2>());
+      };
+      if constexpr (BMAJ) walk(bm_stage);
+      else walk(stage_body);
+    } else if constexpr (BMAJ) {
       for (; kt + 2 < nk; kt++) bm_stage(kt, kt & 1, std::integral_constant<int, 0>());
       if (kt + 1 < nk) {
         bm_stage(kt, kt & 1, std::integral_constant<int, 1>());
@@ -803,6 +842,7 @@ void block_gemm_kernel(const GemmArgs a) {
       }
       stage_body(kt, kt & 1, std::integral_constant<int, 2>());
     }
+    if constexpr (RING) write_ep(0);
     // every wave is done reading the stage buffers (and the scale ring) of this tile
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     barrier();
@@ -810,7 +850,7 @@ void block_gemm_kernel(const GemmArgs a) {
     // ---- next tile's first stage, then this tile's epilogue
     const int64_t em0 = m0, en0 = n0;
     t += nwx;
-    const bool more = t < t_end;
+    const bool more = !RING && t < t_end;  // (a ring's grid has a workgroup per tile)
     if (more) {
       tile_origin(t, m0, n0);
       plan_loads(m0, n0, tl);

@@ -1,0 +1,63 @@
+// Ring tiles: block_gemm_kernel with one small tile per workgroup and three or more stage buffers, for problems
+// whose 256 x 256 or 128 x 128 tiles would leave compute units idle.
+//
+// Such a problem is bound by latency: a workgroup has a compute unit nearly to itself, and its chain of stages
+// (wait, barrier, fragment reads, products, fold) sets the time, K / 128 times over.  So the tile is the smallest
+// that still gives every compute unit work once, each wave gets one or two 32 x 32 blocks (a short chain and a
+// short fold), and two or more stages are always in flight.  Time per 128-channel stage with one workgroup on a
+// compute unit, int8 g128 / int8 per token / fp8 blocks (us): 64 channels x 32 tokens 0.42 / 0.25 / 0.31, 64 x 64
+// 0.45 / 0.28 / 0.36, 128 x 64 0.63 / 0.41 / 0.47, 128 x 128 in eight waves 0.90 / 0.47 / 0.60, against 0.90 / 0.79 /
+// 0.83 for the two-stage 128 x 128 tile of four waves and 1.97 / 1.2 / 1.35 for the 256 x 256 tile.
+#pragma once
+
+#include "gemm_launch.h"
+
+namespace hn {
+
+enum class RingTile { kNone, k64x32, k64x64, k128x64, k128x128 };  // channels x tokens
+
+// The smallest tile that covers the problem in one round of workgroups; 128 x 64 also serves two per compute unit,
+// where it fills the chip better than 128 x 128 tiles that no longer fit one round (300 x 2048 -> 12288: 23.2 -> 18.2
+// us g128, 15.8 -> 13.1 per token).  Larger problems keep the persistent tiles: from two full rounds of 128 x 128 on
+// those move fewer bytes per product (1024 x 3072 -> 12288: 72 us against 85).  GEMM alone, old and new (us):
+//   tokens x K -> N        int8 g128        int8 per token   fp8 blocks
+//   32 x 12288 -> 3072     85.7 -> 41.0     76.5 -> 25.0     80.8 -> 30.3
+//   100 x 3072 -> 3072     21.6 -> 12.5     19.4 -> 8.4      20.2 -> 9.9
+//   200 x 12288 -> 3072    88.9 -> 46.0     76.4 -> 28.0     83.1 -> 36.1
+//   500 x 3072 -> 3072     23.0 -> 17.0     19.9 -> 11.5     21.1 -> 13.4
+//   1024 x 3072 -> 3072    24.7 -> 24.8     20.7 -> 15.1     22.1 -> 18.4
+inline RingTile choose_ring(int64_t M, int64_t N) {
+  const int64_t cus = cu_count();
+  auto tiles = [&](int64_t bn, int64_t bm) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
+  if (tiles(64, 32) <= cus) return RingTile::k64x32;
+  if (tiles(64, 64) <= cus) return RingTile::k64x64;
+  if (tiles(128, 64) <= cus) return RingTile::k128x64;
+  if (tiles(128, 128) <= cus) return RingTile::k128x128;
+  if (tiles(128, 64) <= 2 * cus) return RingTile::k128x64;
+  return RingTile::kNone;
+}
+
+template <int KIND, int EPI, bool G128, int OUT_DT, bool WBLK>
+static int launch_ring_tile(RingTile tile, GemmArgs& a, hipStream_t st) {
+  switch (tile) {
+    case RingTile::k64x32: return launch_cfg<KIND, EPI, G128, 2, 1, 1, 1, OUT_DT, 128, 4, WBLK, 2>(a, st);
+    case RingTile::k64x64: return launch_cfg<KIND, EPI, G128, 2, 2, 1, 1, OUT_DT, 128, 4, WBLK, 2>(a, st);
+    case RingTile::k128x64: return launch_cfg<KIND, EPI, G128, 2, 2, 2, 1, OUT_DT, 128, 3, WBLK, 2>(a, st);
+    default: return launch_cfg<KIND, EPI, G128, 2, 4, 2, 1, OUT_DT, 128, 4, WBLK, 2>(a, st);
+  }
+}
+
+template <int KIND, bool G128, bool WBLK>
+static int launch_ring(GemmArgs& a, int epilogue, int out_dtype, hipStream_t st, bool* taken) {
+  const RingTile tile = choose_ring(a.M, a.N);
+  *taken = tile != RingTile::kNone && (epilogue == HN_EPI_NONE || epilogue == HN_EPI_GELU) &&
+           (out_dtype == HN_DTYPE_BF16 || out_dtype == HN_DTYPE_F16);
+  if (!*taken) return HN_OK;
+  if (epilogue == HN_EPI_NONE)
+    return out_dtype == HN_DTYPE_BF16 ? launch_ring_tile<KIND, HN_EPI_NONE, G128, HN_DTYPE_BF16, WBLK>(tile, a, st)
+                                      : launch_ring_tile<KIND, HN_EPI_NONE, G128, HN_DTYPE_F16, WBLK>(tile, a, st);
+  return out_dtype == HN_DTYPE_BF16 ? launch_ring_tile<KIND, HN_EPI_GELU, G128, HN_DTYPE_BF16, WBLK>(tile, a, st)
+                                    : launch_ring_tile<KIND, HN_EPI_GELU, G128, HN_DTYPE_F16, WBLK>(tile, a, st);
+}
+
+}  // namespace hn
