@@ -3,6 +3,7 @@
 The library is loaded lazily on first use, after torch (whose HIP runtime it binds to).  There is no
 fallback: if the library is missing or a call fails, a RuntimeError says why.
 """
+import contextlib
 import ctypes
 import os
 import threading
@@ -20,6 +21,7 @@ NORM = {"layer": 0, "rms": 1}
 
 _lib = None
 _lock = threading.Lock()
+_SAME_DEVICE = contextlib.nullcontext()
 
 _p = ctypes.c_void_p
 _i64 = ctypes.c_int64
@@ -80,7 +82,7 @@ def lib():
 
 def call(name, *args):
     """Call an entry point; a non-zero status raises RuntimeError with the library's message."""
-    l = lib()
+    l = _lib or lib()
     rc = getattr(l, name)(*args)
     if rc != 0:
         msg = l.hn_last_error().decode(errors="replace")
@@ -94,7 +96,14 @@ def require_device(*tensors):
 
 
 def stream(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The handle of the current stream of t's device (0.1 us; building torch's Stream object for it takes 2)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def on_device(t):
+    """A context with t's device current (null if it is already: entering torch's takes 1.4 us)."""
+    index = t.get_device()
+    return _SAME_DEVICE if torch._C._cuda_getDevice() == index else torch.cuda.device(index)
 
 
 def ptr(t):

@@ -100,8 +100,9 @@ def quantize_activations(x, kind="int8", group=GROUP, rounding="half_away"):
         return q, s
     x = _rows(x)
     _lib.call("hn_quantize_act", x.data_ptr(), _lib.dtype_code(x), x.stride(0), m, k, g, _lib.KIND[kind],
-              _lib.ROUND[rounding], q.data_ptr(), q.stride(0), s.data_ptr(), s.stride(0), _lib.stream(x))
-    trust_scales(s)
+              _lib.ROUND[rounding], q.data_ptr(), k, s.data_ptr(), k // g, _lib.stream(x))
+    if kind == "fp8":  # (only the fp8 block scales' running sum asks for a verdict)
+        trust_scales(s)
     return q, s
 
 
@@ -350,8 +351,7 @@ def block_linear(x, qw, sw, bias=None, kind="int8", rounding="half_away"):
     [ceil(N/128), K/128] (one row per 128 output channels) are taken as they are.  One library call
     (hn_block_linear) quantizes into a workspace and runs the GEMM.  `rounding` (an addition to the
     reference's signature): "half_even" rounds the int8 activation codes half to even."""
-    shape = x.shape
-    x2 = x.reshape(-1, shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if not x2.is_contiguous():
         x2 = x2.contiguous()
     m, k = x2.shape
@@ -368,10 +368,10 @@ def block_linear(x, qw, sw, bias=None, kind="int8", rounding="half_away"):
     sw, sw_rows, gemm_group, groups = _layout(sw, n, k, kind, k // group)
     if gemm_group != group:
         # per-token scales over a K the int32 sum cannot hold: quantize per token, fold per group
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x):
             qa, sa = quantize_activations(x2, kind, None, rounding)
             out = block_gemm(qa, sa, qw, sw, bias, x.dtype, kind)
-        return out.reshape(*shape[:-1], n)
+        return out.reshape(*x.shape[:-1], n)
     if x2.dtype not in _lib.DTYPE:
         x2 = x2.float()
     x2 = _rows(x2)
@@ -379,15 +379,17 @@ def block_linear(x, qw, sw, bias=None, kind="int8", rounding="half_away"):
     qw = _rows(qw)
     if bias is not None and not bias.is_contiguous():
         bias = bias.contiguous()
-    out = torch.empty((m, n), device=x.device, dtype=x.dtype if x.dtype in _lib.DTYPE else torch.float32)
+    out = torch.empty((m, n), device=x.device, dtype=x2.dtype)
     nbytes = _lib.lib().hn_block_linear_workspace_bytes(m, k, group)
     ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x):
         _lib.call("hn_block_linear", x2.data_ptr(), _lib.dtype_code(x2), x2.stride(0), m, k, group, _lib.KIND[kind],
                   _lib.ROUND[rounding], qw.data_ptr(), qw.stride(0), sw.data_ptr(), sw.stride(0), sw_rows,
                   _lib.ptr(bias), _lib.dtype_code(bias) if bias is not None else 0, n, out.data_ptr(),
-                  _lib.dtype_code(out), out.stride(0), ws.data_ptr(), nbytes, _lib.stream(x2))
-    return out.reshape(*shape[:-1], n).to(x.dtype)
+                  _lib.dtype_code(out), n, ws.data_ptr(), nbytes, _lib.stream(x2))
+    if x.dim() != 2:
+        out = out.reshape(*x.shape[:-1], n)
+    return out if out.dtype == x.dtype else out.to(x.dtype)
 
 
 def int8_g128_linear(x, qw, sw, bias=None):

@@ -17,7 +17,7 @@ import dataclasses
 import torch
 import torch.nn.functional as F
 
-from . import kernels
+from . import _lib, kernels
 
 try:
     import comfy.model_management  # noqa: F401
@@ -291,7 +291,7 @@ def swiglu_mlp(x, gate_up, down, bias=None):
     x2 = x.reshape(-1, k)
     if x2.dtype not in (torch.bfloat16, torch.float16, torch.float32):
         x2 = x2.to(torch.bfloat16)
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x):
         qa, sa = kernels.quantize_activations(x2, "fp8")
         hq, hs = kernels.block_gemm(qa, sa, q_gu, s_gu, kind="fp8", epilogue="swiglu_quant")
         y = kernels.block_gemm(hq, hs, q_d, s_d, bias, out_dtype=x.dtype, kind="fp8")
