@@ -161,13 +161,52 @@ static int launch_skinny_mode(GemmArgs& a, int epilogue, int out_dtype, hipStrea
   return launch_skinny_epi<4, MODE>(a, epilogue, out_dtype, st);
 }
 
-}  // namespace hn
+// The same from a 16-bit source (run_linear's M <= 4): codes and scales in LDS, outputs in the source's dtype.
+template <int MT, int MODE, int DT>
+static int launch_skinny_x(GemmArgs& a, int rounding, hipStream_t st) {
+  constexpr int64_t ROWS = kSkinnyRows * kSkinnyWaves;
+  const int64_t grid = (a.N + ROWS - 1) / ROWS;
+  if (grid > 0x7fffffff) {
+    set_error("hn_block_gemm: problem too large (N=%lld)", (long long)a.N);
+    return HN_ERR_UNSUPPORTED;
+  }
+  const dim3 g((unsigned)grid), b(kSkinnyWaves * 64);
+  const unsigned lds = (unsigned)(a.M * a.K + a.M * (MODE == 0 ? 1 : a.K / 128) * 4);
+  if (rounding == HN_ROUND_HALF_EVEN)
+    hipLaunchKernelGGL((skinny_gemm_kernel<MT, MODE, HN_EPI_NONE, DT, DT, HN_ROUND_HALF_EVEN>), g, b, lds, st, a);
+  else
+    hipLaunchKernelGGL((skinny_gemm_kernel<MT, MODE, HN_EPI_NONE, DT, DT, HN_ROUND_HALF_AWAY>), g, b, lds, st, a);
+  return HN_LAUNCH_CHECK("skinny_gemm_kernel");
+}
 
-extern "C" int hn_block_gemm(const void* qa, int64_t lda, const float* sa, int64_t ldsa, const void* qw, int64_t ldw,
-                             const float* sw, int64_t ldsw, int64_t sw_rows, const void* bias, int bias_dtype, int64_t M, int64_t N,
-                             int64_t K, int64_t group, int kind, int epilogue, void* out, int out_dtype, int64_t ldo,
-                             float* qs, int64_t ldqs, void* stream) {
-  using namespace hn;
+template <int MODE, int DT>
+static int launch_skinny_x_mode(GemmArgs& a, int rounding, hipStream_t st) {
+  if (a.M == 1) return launch_skinny_x<1, MODE, DT>(a, rounding, st);
+  if (a.M == 2) return launch_skinny_x<2, MODE, DT>(a, rounding, st);
+  return launch_skinny_x<4, MODE, DT>(a, rounding, st);
+}
+
+template <int DT>
+static int launch_skinny_x_dt(GemmArgs& a, bool g128, int rounding, hipStream_t st) {
+  if (!g128) return launch_skinny_x_mode<0, DT>(a, rounding, st);
+  if (a.sw_rows == 128) return launch_skinny_x_mode<2, DT>(a, rounding, st);
+  return launch_skinny_x_mode<1, DT>(a, rounding, st);
+}
+
+// Up to four rows whose codes fit 48 KB of LDS (three workgroups on a compute unit), 16-byte aligned, in a quantization
+// that the quantizer takes.  3072 -> 18432 at one row: quantizer and GEMM 2.6 + 11.5 us.
+bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t group, int kind,
+                         int rounding, int out_dtype) {
+  return M > 0 && M <= kSkinnyMaxM && kind == HN_KIND_INT8 && (x_dtype == HN_DTYPE_BF16 || x_dtype == HN_DTYPE_F16) &&
+         out_dtype == x_dtype && M * K <= 49152 && (group == 128 || K <= 16384) && ldx >= K && ldx % 8 == 0 &&
+         ((uintptr_t)x & 15) == 0 && (rounding == HN_ROUND_HALF_AWAY || rounding == HN_ROUND_HALF_EVEN);
+}
+
+// hn_block_gemm, or (x given, skinny_takes_source) the linear of x itself; qa and sa are then not read.
+static int block_gemm_impl(const void* x, int64_t ldx, int rounding, const void* qa, int64_t lda, const float* sa,
+                           int64_t ldsa, const void* qw, int64_t ldw, const float* sw, int64_t ldsw, int64_t sw_rows,
+                           const void* bias, int bias_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int kind,
+                           int epilogue, void* out, int out_dtype, int64_t ldo, float* qs, int64_t ldqs, void* stream) {
   HN_REQUIRE(M >= 0 && N > 0 && K > 0, "hn_block_gemm: bad shape M=%lld N=%lld K=%lld", (long long)M, (long long)N,
              (long long)K);
   HN_REQUIRE(K % 128 == 0, "hn_block_gemm: K=%lld is not a multiple of 128", (long long)K);
@@ -217,6 +256,12 @@ extern "C" int hn_block_gemm(const void* qa, int64_t lda, const float* sa, int64
   // per-token mode also serves a single-group K == 128 problem with one scale row per channel
   const bool g128 = group == 128 && (K != 128 || sw_rows == 128);
   if (epilogue == HN_EPI_ACC32) return launch_group<HN_KIND_INT8, HN_EPI_ACC32, HN_DTYPE_BF16>(a, false, st);
+  if (x != nullptr) {
+    a.x = (const uint16_t*)x;
+    a.ldx = ldx;
+    return out_dtype == HN_DTYPE_BF16 ? launch_skinny_x_dt<HN_DTYPE_BF16>(a, g128, rounding, st)
+                                      : launch_skinny_x_dt<HN_DTYPE_F16>(a, g128, rounding, st);
+  }
   if (kind == HN_KIND_INT8 && M <= kSkinnyMaxM && (epilogue == HN_EPI_NONE || epilogue == HN_EPI_GELU)) {
     if (!g128) return launch_skinny_mode<0>(a, epilogue, out_dtype, st);
     if (sw_rows == 128) return launch_skinny_mode<2>(a, epilogue, out_dtype, st);
@@ -232,6 +277,25 @@ extern "C" int hn_block_gemm(const void* qa, int64_t lda, const float* sa, int64
   }
   if (kind == HN_KIND_INT8) return launch_kind<HN_KIND_INT8>(a, g128, epilogue, out_dtype, st);
   return launch_kind<HN_KIND_FP8>(a, g128, epilogue, out_dtype, st);
+}
+
+
+int skinny_linear(const void* x, int64_t ldx, int rounding, const void* qa, const float* sa, const void* qw, int64_t ldw,
+                  const float* sw, int64_t ldsw, int64_t sw_rows, const void* bias, int bias_dtype, int64_t M, int64_t N,
+                  int64_t K, int64_t group, void* out, int out_dtype, int64_t ldo, void* stream) {
+  return block_gemm_impl(x, ldx, rounding, qa, K, sa, K / group, qw, ldw, sw, ldsw, sw_rows, bias, bias_dtype, M, N, K, group,
+                         HN_KIND_INT8, HN_EPI_NONE, out, out_dtype, ldo, nullptr, 0, stream);
+}
+
+}  // namespace hn
+
+extern "C" int hn_block_gemm(const void* qa, int64_t lda, const float* sa, int64_t ldsa, const void* qw, int64_t ldw,
+                             const float* sw, int64_t ldsw, int64_t sw_rows, const void* bias, int bias_dtype, int64_t M, int64_t N,
+                             int64_t K, int64_t group, int kind, int epilogue, void* out, int out_dtype, int64_t ldo,
+                             float* qs, int64_t ldqs, void* stream) {
+  using namespace hn;
+  return block_gemm_impl(nullptr, 0, 0, qa, lda, sa, ldsa, qw, ldw, sw, ldsw, sw_rows, bias, bias_dtype, M, N, K, group, kind,
+                         epilogue, out, out_dtype, ldo, qs, ldqs, stream);
 }
 
 static int qkv_heads_impl(const void* qa, int64_t lda, const float* sa, int64_t ldsa, const void* qw, int64_t ldw,

@@ -72,6 +72,9 @@ struct GemmArgs {
   // token l at key hm_loff + l (hm_L % 32 == 0, hm_loff % 16 == 0)
   uint16_t* hm_vt;
   int64_t hm_svb, hm_svh, hm_svd;
+  // the skinny kernel's source: 16-bit x [M, K] with row stride ldx, instead of codes and scales
+  const uint16_t* x;
+  int64_t ldx;
 };
 
 // Internal epilogue id of the head-major QKV projection (entry point hn_qkv_heads).

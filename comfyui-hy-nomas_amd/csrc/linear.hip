@@ -25,13 +25,17 @@ int check_linear(const char* who, const void* x, int64_t M, int64_t N, int64_t K
   return HN_OK;
 }
 
-// Quantize x into the workspace, then run the GEMM from it (both enqueued on `stream`).
+// Quantize x into the workspace, then run the GEMM from it (both enqueued on `stream`); a few rows of 16-bit x go to the
+// skinny kernel, which quantizes them itself (gemm.hip).
 int run_linear(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t group, int kind, int rounding,
                const void* qw, int64_t ldw, const float* sw, int64_t ldsw, int64_t sw_rows, const void* bias,
                int bias_dtype, int64_t N, void* out, int out_dtype, int64_t ldo, uint8_t* ws, void* stream) {
   if (M == 0) return HN_OK;
   float* s = reinterpret_cast<float*>(ws + linear_scales_offset(M, K));
   const int64_t ng = K / group;
+  if (skinny_takes_source(x, x_dtype, ldx, M, K, group, kind, rounding, out_dtype))
+    return skinny_linear(x, ldx, rounding, ws, s, qw, ldw, sw, ldsw, sw_rows, bias, bias_dtype, M, N, K, group, out, out_dtype,
+                         ldo, stream);
   int rc = hn_quantize_act(x, x_dtype, ldx, M, K, group, kind, rounding, ws, K, s, ng, stream);
   if (rc != HN_OK) return rc;
   return hn_block_gemm(ws, K, s, ng, qw, ldw, sw, ldsw, sw_rows, bias, bias_dtype, M, N, K, group, kind, HN_EPI_NONE,

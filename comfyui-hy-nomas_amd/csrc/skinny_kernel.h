@@ -10,9 +10,14 @@
 //     folded in group order, acc = fma(float(part) * sa[m, g], sw[n, g], acc) (block weight scales:
 //     acc = fma(float(part), sa[m, g] * sw[n / 128, g], acc)), from the partials read lane by lane;
 //   * + bias (absent: -0.0), optional GELU, the same output conversion.
+//
+// With a source (SRC, the linear's 16-bit x) the kernel quantizes it itself: each workgroup forms the codes and scales
+// of its M rows in LDS, with the quantizer's own arithmetic, while its first weights are on the way.  At most 48 KB
+// of codes, read from L2 by every workgroup; in return the quantizer's launch and the codes' trip through memory go.
 #pragma once
 
 #include "gemm_kernel.h"
+#include "quant_codes.h"
 
 namespace hn {
 
@@ -20,13 +25,67 @@ constexpr int kSkinnyRows = 4;     // weight rows per wave
 constexpr int kSkinnyWaves = 4;    // waves per workgroup
 constexpr int kSkinnyMaxM = 4;
 
+// The codes and scales of the M rows of a.x into LDS, by the whole workgroup: as quant_g128_kernel (16 lanes a group) or,
+// with one scale per token, as quant_row_kernel (the row's absmax over the workgroup, then the codes).
+template <bool PER_TOKEN, int DT, int ROUND>
+__device__ __forceinline__ void quantize_rows(const GemmArgs& a, uint8_t* codes, float* scales) {
+  constexpr int T = kSkinnyWaves * 64;
+  __shared__ float peaks[kSkinnyWaves][kSkinnyMaxM];
+  const int tid = threadIdx.x, M = (int)a.M, K = (int)a.K;
+  auto widen = [&](int m, int c, float* f) __attribute__((always_inline)) {  // values 8 c .. 8 c + 7 of row m
+    In<DT>::widen8(*reinterpret_cast<const uint4*>(a.x + m * a.ldx + 8 * c), f);
+  };
+  if constexpr (PER_TOKEN) {
+    for (int m = 0; m < M; m++) {
+      float peak = 0.0f;
+      for (int c = tid; c < K / 8; c += T) {
+        float f[8];
+        widen(m, c, f);
+#pragma unroll
+        for (int i = 0; i < 8; i++) peak = __builtin_fmaxf(peak, __builtin_fabsf(f[i]));
+      }
+      peak = wave_max_nonneg(peak);
+      if ((tid & 63) == 0) peaks[tid >> 6][m] = peak;
+    }
+    __syncthreads();
+    for (int m = 0; m < M; m++) {
+      float peak = peaks[0][m];
+#pragma unroll
+      for (int w = 1; w < kSkinnyWaves; w++) peak = __builtin_fmaxf(peak, peaks[w][m]);
+      float sc = 0.0f;
+      for (int c = tid; c < K / 8; c += T) {
+        float f[8];
+        widen(m, c, f);
+        *reinterpret_cast<uint2*>(codes + m * K + 8 * c) = encode8_group<DT, HN_KIND_INT8, ROUND>(f, peak, sc);
+      }
+      if (tid == 0) scales[m] = sc;
+    }
+  } else {
+    const int G = K / 128;
+    for (int u = tid >> 4; u < M * G; u += T / 16) {
+      const int m = u / G, g = u - m * G;
+      float f[8], sc;
+      widen(m, g * 16 + (tid & 15), f);
+      float peak = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; i++) peak = __builtin_fmaxf(peak, __builtin_fabsf(f[i]));
+      peak = row16_max_nonneg(peak);
+      *reinterpret_cast<uint2*>(codes + m * K + (g * 16 + (tid & 15)) * 8) = encode8_group<DT, HN_KIND_INT8, ROUND>(f, peak, sc);
+      if ((tid & 15) == 0) scales[u] = sc;
+    }
+  }
+  __syncthreads();
+}
+
 // MODE 0: per-token x per-channel (whole-K int32); 1: g128 with one weight-scale row per channel;
-// 2: g128 with one weight-scale row per 128 channels.
-template <int MT, int MODE, int EPI, int OUT_DT>
+// 2: g128 with one weight-scale row per 128 channels.  SRC: the dtype of a.x, or -1 for the codes a.qa with scales a.sa.
+template <int MT, int MODE, int EPI, int OUT_DT, int SRC = -1, int ROUND = HN_ROUND_HALF_AWAY>
 __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_kernel(const GemmArgs a) {
+  constexpr bool FROM_X = SRC >= 0;
+  extern __shared__ __align__(16) uint8_t xq[];  // FROM_X: codes [M][K], then scales [M][G or 1]
   const int lane = threadIdx.x & 63;
   const int64_t n0 = ((int64_t)blockIdx.x * kSkinnyWaves + (threadIdx.x >> 6)) * kSkinnyRows;
-  if (n0 >= a.N) return;  // whole wave (the kernel has no workgroup barrier)
+  if (!FROM_X && n0 >= a.N) return;  // whole wave (no workgroup barrier without a source)
   const int G = (int)(a.K / 128);
   const int steps = (G + 7) / 8;
   const int M = (int)a.M;
@@ -36,7 +95,9 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_kernel(const Ge
   for (int r = 0; r < kSkinnyRows; r++) wrow[r] = a.qw + (n0 + r < a.N ? n0 + r : a.N - 1) * a.ldw;
   const uint8_t* xrow[MT];
 #pragma unroll
-  for (int m = 0; m < MT; m++) xrow[m] = a.qa + (int64_t)(m < M ? m : M - 1) * a.lda;
+  for (int m = 0; m < MT; m++)
+    xrow[m] = FROM_X ? xq + (m < M ? m : M - 1) * (int)a.K : a.qa + (int64_t)(m < M ? m : M - 1) * a.lda;
+  float* xs = reinterpret_cast<float*>(xq + M * (int)a.K);
 
   int32_t acc32[kSkinnyRows][MT];
   float facc[kSkinnyRows][MT];
@@ -57,24 +118,36 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_kernel(const Ge
     swrow[r] = MODE == 2 ? a.sw + (n / 128) * a.ldsw : a.sw + n * a.ldsw;
   }
 #pragma unroll
-  for (int m = 0; m < MT; m++) sarow[m] = a.sa + (int64_t)(m < M ? m : M - 1) * a.ldsa;
+  for (int m = 0; m < MT; m++)
+    sarow[m] = FROM_X ? xs + (m < M ? m : M - 1) * (MODE == 0 ? 1 : G) : a.sa + (int64_t)(m < M ? m : M - 1) * a.ldsa;
   v4i wv[2][kSkinnyRows], xv[2][MT];
   float swl[2][kSkinnyRows], sal[2][MT];
-  auto load = [&](int s, int buf) __attribute__((always_inline)) {
+  auto load_w = [&](int s, int buf) __attribute__((always_inline)) {
     const bool ok = 8 * s + (lane >> 3) < G;
     const uint32_t off = (uint32_t)s * 1024u + (uint32_t)lane * 16u;
 #pragma unroll
     for (int r = 0; r < kSkinnyRows; r++)
       wv[buf][r] = ok ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(wrow[r] + off)) : v4i{0, 0, 0, 0};
+    if constexpr (MODE != 0) {
+      const int gl = min(8 * s + (lane >> 3), G - 1);
+#pragma unroll
+      for (int r = 0; r < kSkinnyRows; r++) swl[buf][r] = swrow[r][gl];
+    }
+  };
+  auto load_x = [&](int s, int buf) __attribute__((always_inline)) {
+    const bool ok = 8 * s + (lane >> 3) < G;
+    const uint32_t off = (uint32_t)s * 1024u + (uint32_t)lane * 16u;
 #pragma unroll
     for (int m = 0; m < MT; m++) xv[buf][m] = ok ? *reinterpret_cast<const v4i*>(xrow[m] + off) : v4i{0, 0, 0, 0};
     if constexpr (MODE != 0) {
       const int gl = min(8 * s + (lane >> 3), G - 1);
 #pragma unroll
-      for (int r = 0; r < kSkinnyRows; r++) swl[buf][r] = swrow[r][gl];
-#pragma unroll
       for (int m = 0; m < MT; m++) sal[buf][m] = sarow[m][gl];
     }
+  };
+  auto load = [&](int s, int buf) __attribute__((always_inline)) {
+    load_w(s, buf);
+    load_x(s, buf);
   };
   auto compute = [&](int s, int buf) __attribute__((always_inline)) {
     float t[kSkinnyRows][MT], f[kSkinnyRows][MT];
@@ -128,7 +201,12 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_kernel(const Ge
       }
     }
   };
-  load(0, 0);
+  load_w(0, 0);
+  if constexpr (FROM_X) {
+    quantize_rows<MODE == 0, SRC, ROUND>(a, xq, xs);
+    if (n0 >= a.N) return;
+  }
+  load_x(0, 0);
   int s = 0;
   for (; s + 1 < steps; s += 2) {
     load(s + 1, 1);
@@ -151,7 +229,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void skinny_gemm_kernel(const Ge
         v += __shfl_xor(v, 16);
         v += __shfl_xor(v, 32);
         const int64_t n = n0 + r < a.N ? n0 + r : a.N - 1;
-        facc[r][m] = __builtin_fmaf((float)v * a.sa[(int64_t)(m < M ? m : M - 1) * a.ldsa], a.sw[n * a.ldsw], 0.0f);
+        facc[r][m] = __builtin_fmaf((float)v * sarow[m][0], a.sw[n * a.ldsw], 0.0f);
       }
   }
   // every lane holds the same results; lane r * MT + m stores output (m, n0 + r)
