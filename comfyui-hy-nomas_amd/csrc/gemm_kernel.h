@@ -439,6 +439,21 @@ void block_gemm_kernel(const GemmArgs a) {
   // (it needs two token blocks: the next channel block's weight fragments are read during the last one)
   constexpr bool BMAJ = G128 && !RESCALE && !WBLK && STAGES_PER_GROUP == 1 && TM >= 2;
   Frag fbs[BMAJ ? TM : 1][BMAJ ? SLICES : 1], fas[BMAJ ? SLICES : 1];
+  // AHEAD: ring tiles that read a whole stage's fragments one stage ahead (ring_stage), in two register sets.  Not the
+  // waves of two channel blocks, which that makes up to 8 % slower (per token, fp8) or leaves as they are (g128).
+  constexpr bool AHEAD = RING && TN == 1;
+  static_assert(!RING || !BMAJ, "ring tiles have one token block a wave");
+  static_assert(!AHEAD || (STAGES_PER_GROUP == 1 && !(WBLK && !RESCALE)), "ring_stage");
+  Frag ra[AHEAD ? 2 : 1][AHEAD ? SLICES : 1][AHEAD ? TN : 1], rb[AHEAD ? 2 : 1][AHEAD ? SLICES : 1][AHEAD ? TM : 1];
+  auto read_stage = [&](int set, const char* stage_base) __attribute__((always_inline)) {
+#pragma unroll
+    for (int s = 0; s < SLICES; s++) {
+#pragma unroll
+      for (int i = 0; i < TN; i++) ra[set][s][i] = MF::template load<BK>(stage_base, wrow_n + i * 32, s, lane);
+#pragma unroll
+      for (int j = 0; j < TM; j++) rb[set][s][j] = MF::template load<BK>(stage_base + A_BYTES, wrow_m + j * 32, s, lane);
+    }
+  };
 
   // The tile's epilogue operands (per-channel weight scale and bias, per-token activation scale), parked in
   // LDS for the epilogue.  Rows and channels past the edge take the last valid one; an absent bias reads as
@@ -554,7 +569,9 @@ void block_gemm_kernel(const GemmArgs a) {
     barrier();
     if constexpr (!EARLY_EP && !RING) write_ep(0);
     if (!RING && 1 < nk) issue_stage(1, 1);
-    if constexpr (BMAJ) {
+    if constexpr (AHEAD) {
+      read_stage(0, smem + SCR);
+    } else if constexpr (BMAJ) {
 #pragma unroll
       for (int j = 0; j < TM; j++)
 #pragma unroll
@@ -596,9 +613,9 @@ void block_gemm_kernel(const GemmArgs a) {
     // One K stage (kt, in buffer `buf`).  The schedule is pinned with scheduling barriers (address
     // arithmetic may still move): each slice issues the next slice's fragment reads right after its
     // first products, so they land while the matrix core works.  The last slice holds the stage
-    // barrier; after it the next stage's first fragments are read and the direct loads of stage kt + NS
+    // barrier; after it the next stage's first fragments are read and the direct loads of stage kt + 2
     // are interleaved with the slice's remaining products, so the matrix core is fed while the loads
-    // queue.  MODE 0: barrier and loads; 1: barrier, no loads (stage kt + NS does not exist); 2: the
+    // queue.  MODE 0: barrier and loads; 1: barrier, no loads (stage kt + 2 does not exist); 2: the
     // tile's last stage (neither).
     // Weight rows multiplied before the barrier.  Per-token tiles issue all of the last slice's products
     // after it (1.7 % faster over the DiT stack); the g128 and block-scale tiles keep one row before it
@@ -655,7 +672,7 @@ void block_gemm_kernel(const GemmArgs a) {
           // stage kt + 1 (the oldest loads in flight) has landed for this wave and its reads of stage kt
           // are complete; the barrier publishes both facts, then stage kt + NS may refill `buf`
           if constexpr (MODE == 0 || !RING) wait_vmcnt<LOADS*(NS - 2)>();
-          else wait_stages(nk - 2 - kt);
+          else wait_stages(min(nk - 2 - kt, NS - 2));
           __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
           barrier();
           __builtin_amdgcn_sched_barrier(0);
@@ -763,11 +780,11 @@ void block_gemm_kernel(const GemmArgs a) {
     // its reads before its share of the fold: the group's scales after the first product, the next channel
     // block's weight fragments (slice by slice, as the last token block releases them).  The last channel
     // block follows the stage barrier, reads the next stage's activation fragments as its products release
-    // them, and spreads the direct loads of stage kt + NS over its products.
+    // them, and spreads the direct loads of stage kt + 2 over its products.
     auto bm_stage = [&](int kt, int buf, auto mode_c) __attribute__((always_inline)) {
       constexpr int MODE = decltype(mode_c)::value;
       const char* stage = smem + SCR + buf * STAGE;
-      const char* next = smem + SCR + next_buf(buf) * STAGE;
+      const char* next = smem + SCR + (buf ^ 1) * STAGE;
       // the previous group's last block is folded during this stage's first block, with that group's scales
       const float p_sa = c_sa[TM - 1], p_sw = c_sw[TN - 1];
       static_assert(NB % 2 == 0, "blocks alternate between the two partial sets, block 0 in set 0");
@@ -776,10 +793,9 @@ void block_gemm_kernel(const GemmArgs a) {
         constexpr int pb = (b + NB - 1) % NB, pi = pb / TM, pj = pb % TM;  // the block folded meanwhile
         if constexpr (b == LAST && MODE != 2) {
           // every wave's reads of this stage are done and stage kt + 1 has landed: the barrier publishes
-          // both, then the next stage's fragments are read and stage kt + NS refills `buf`
+          // both, then the next stage's fragments are read and stage kt + 2 refills `buf`
           __builtin_amdgcn_sched_barrier(0);
-          if constexpr (MODE == 0 || !RING) wait_vmcnt<LOADS*(NS - 2)>();
-          else wait_stages(nk - 2 - kt);
+          wait_vmcnt<0>();
           __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
           barrier();
           __builtin_amdgcn_sched_barrier(0);
@@ -799,7 +815,7 @@ void block_gemm_kernel(const GemmArgs a) {
             if constexpr (MODE == 0) {
               constexpr int slot = j * SLICES + s, SLOTS = TM * SLICES;
 #pragma unroll
-              for (int q = slot * LOADS / SLOTS; q < (slot + 1) * LOADS / SLOTS; q++) issue_load(kt + NS, buf, q);
+              for (int q = slot * LOADS / SLOTS; q < (slot + 1) * LOADS / SLOTS; q++) issue_load(kt + 2, buf, q);
             }
           }
           __builtin_amdgcn_sched_barrier(0);
@@ -811,18 +827,109 @@ void block_gemm_kernel(const GemmArgs a) {
         });
       });
     };
+    // One stage of an AHEAD ring tile (kt, in buffer `buf`, its fragments in register set SET).  A stage's fragments are
+    // all read one stage ahead: their latency passes under the products and the fold, and the stage's own buffer is free
+    // for stage kt + NS at its one barrier.  What remains is the direct loads' rate per compute unit (28 B a clock: 430
+    // clocks for the 12 KB of a 64 x 32 stage).  64 x 32 and 64 x 64 tiles, slice by slice and so (us): 100 x 12288 -> 3072
+    // g128 38.9 -> 32.7, 300 x 8192 -> 2048 29.2 / 19.1 / 24.4 -> 24.0 / 15.6 / 20.1 (g128 / per token / fp8 blocks),
+    // 100 x 3072 -> 3072 12.6 / 8.5 / 9.9 -> 10.9 / 7.5 / 9.2.  MODE 0: loads
+    // where stage kt + NS exists; 1: the same near the end, with fewer stages in flight; 2: the tile's last stage.
+    auto ring_stage = [&](int kt, int buf, auto set_c, auto mode_c) __attribute__((always_inline)) {
+      constexpr int SET = decltype(set_c)::value, MODE = decltype(mode_c)::value;
+      constexpr int MFMAS = SLICES * TN * TM;
+      if constexpr (MODE != 2) {
+        // stage kt + 1 has landed for this wave, and its reads of stage kt are complete
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (MODE == 0) wait_vmcnt<LOADS*(NS - 2)>();
+        else wait_stages(min(nk - 2 - kt, NS - 2));
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+        barrier();
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      float sam[TM], swc[TN], rs[TM];
+      if constexpr (G128) {
+        const float* sc = reinterpret_cast<const float*>(smem + (kt % (NS + 1)) * SC_BYTES);
+#pragma unroll
+        for (int j = 0; j < TM; j++) sam[j] = sc[BN + wrow_m + j * 32];
+        if constexpr (WBLK) {
+          swc[0] = sc[wn * TN * 32];
+        } else {  // the lane's DPP source of each channel block's scales (as in stage_body)
+#pragma unroll
+          for (int i = 0; i < TN; i++)
+            swc[i] = sc[wn * TN * 32 + i * 32 + ((lane & 15) >> 2) * 8 + (lane >> 5) * 4 + (lane & 3)];
+        }
+      }
+      if constexpr (MODE != 2) {
+        read_stage(SET ^ 1, smem + SCR + next_buf(buf) * STAGE);
+        if (MODE == 0 || kt + NS < nk) issue_stage(kt + NS, buf);
+      }
+      if constexpr (RESCALE) {  // as in stage_body: each block moves to this group's scale product
+#pragma unroll
+        for (int j = 0; j < TM; j++) {
+          const float den = sam[j] * swc[0];
+          const float r0 = __builtin_amdgcn_rcpf(den);
+          const float r = __builtin_fmaf(__builtin_fmaf(-den, r0, 1.0f), r0, r0);
+          rs[j] = kt > 0 ? ss_last[j] * r : 1.0f;
+          ss_last[j] = den;
+        }
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+          for (int j = 0; j < TM; j++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) acc[i][j][r] *= rs[j];
+      }
+#pragma unroll
+      for (int s = 0; s < SLICES; s++)
+#pragma unroll
+        for (int i = 0; i < TN; i++)
+#pragma unroll
+          for (int j = 0; j < TM; j++) {
+            if (FRESH && s == 0) acc[i][j] = MF::run(ra[SET][s][i], rb[SET][s][j], Acc{});
+            else acc[i][j] = MF::run(ra[SET][s][i], rb[SET][s][j], acc[i][j]);
+          }
+      if constexpr (MODE == 0) {  // the fragment reads first, then products and loads alternating
+        __builtin_amdgcn_sched_group_barrier(0x100, 64, 0);
+#pragma unroll
+        for (int r = 0; r < MFMAS; r++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x020, (LOADS + MFMAS - 1) / MFMAS, 0);
+        }
+      }
+      if constexpr (G128 && !RESCALE) {
+#pragma unroll
+        for (int j = 0; j < TM; j++)
+#pragma unroll
+          for (int i = 0; i < TN; i++)
+            fold_row_bcast(facc[i][j], acc[i][j], sam[j], swc[i], std::make_integer_sequence<int, 16>());
+      }
+    };
     // stages kt = 0 .. nk - 1, each in the buffer after the last one's: MODE 0 while stage kt + NS exists, then
     // MODE 1 and, for the last stage, MODE 2
     int kt = 0;
-    if constexpr (RING) {
+    if constexpr (AHEAD) {
       int buf = 0;
-      auto walk = [&](auto&& stage_fn) __attribute__((always_inline)) {
-        for (; kt + NS < nk; kt++, buf = next_buf(buf)) stage_fn(kt, buf, std::integral_constant<int, 0>());
-        for (; kt + 1 < nk; kt++, buf = next_buf(buf)) stage_fn(kt, buf, std::integral_constant<int, 1>());
-        stage_fn(kt, buf, std::integral_constant<int, 2>());
+      // by twos, so that the fragment set of a stage is a constant
+      auto two = [&](auto mode_c) __attribute__((always_inline)) {
+        ring_stage(kt, buf, std::integral_constant<int, 0>(), mode_c);
+        buf = next_buf(buf);
+        ring_stage(kt + 1, buf, std::integral_constant<int, 1>(), mode_c);
+        buf = next_buf(buf);
+        kt += 2;
       };
-      if constexpr (BMAJ) walk(bm_stage);
-      else walk(stage_body);
+      while (kt + 1 + NS < nk) two(std::integral_constant<int, 0>());
+      while (kt + 2 < nk) two(std::integral_constant<int, 1>());
+      if (kt + 1 < nk) {
+        ring_stage(kt, buf, std::integral_constant<int, 0>(), std::integral_constant<int, 1>());
+        ring_stage(kt + 1, next_buf(buf), std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+      } else {
+        ring_stage(kt, buf, std::integral_constant<int, 0>(), std::integral_constant<int, 2>());
+      }
+    } else if constexpr (RING) {
+      int buf = 0;
+      for (; kt + NS < nk; kt++, buf = next_buf(buf)) stage_body(kt, buf, std::integral_constant<int, 0>());
+      for (; kt + 1 < nk; kt++, buf = next_buf(buf)) stage_body(kt, buf, std::integral_constant<int, 1>());
+      stage_body(kt, buf, std::integral_constant<int, 2>());
     } else if constexpr (BMAJ) {
       for (; kt + 2 < nk; kt++) bm_stage(kt, kt & 1, std::integral_constant<int, 0>());
       if (kt + 1 < nk) {

@@ -21,9 +21,9 @@ enum class RingTile { kNone, k64x32, k64x64, k128x64, k128x128 };  // channels x
 // us g128, 15.8 -> 13.1 per token).  Larger problems keep the persistent tiles: from two full rounds of 128 x 128 on
 // those move fewer bytes per product (1024 x 3072 -> 12288: 72 us against 85).  GEMM alone, old and new (us):
 //   tokens x K -> N        int8 g128        int8 per token   fp8 blocks
-//   32 x 12288 -> 3072     85.7 -> 41.0     76.5 -> 25.0     80.8 -> 30.3
-//   100 x 3072 -> 3072     21.6 -> 12.5     19.4 -> 8.4      20.2 -> 9.9
-//   200 x 12288 -> 3072    88.9 -> 46.0     76.4 -> 28.0     83.1 -> 36.1
+//   32 x 12288 -> 3072     85.7 -> 39.1     76.5 -> 24.7     80.8 -> 30.4
+//   100 x 3072 -> 3072     21.6 -> 10.9     19.4 -> 7.5      20.2 -> 9.2
+//   200 x 12288 -> 3072    88.9 -> 43.6     76.4 -> 26.9     83.1 -> 32.6
 //   500 x 3072 -> 3072     23.0 -> 17.0     19.9 -> 11.5     21.1 -> 13.4
 //   1024 x 3072 -> 3072    24.7 -> 24.8     20.7 -> 15.1     22.1 -> 18.4
 inline RingTile choose_ring(int64_t M, int64_t N) {
