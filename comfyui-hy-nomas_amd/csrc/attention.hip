@@ -89,9 +89,11 @@ struct AttnArgs {
   int H;
   float scale_log2;       // softmax scale times log2(e): the scores are exponentiated base 2
   int qblocks;            // query blocks of one (batch, head)
-  int splits;             // workgroups that share one query block's keys, each a contiguous range of its tiles
-  float4* po;             // splits > 1: unnormalized partial outputs [unit][32 chunks of 4 dims][128 queries]
-  float2* pml;            // and their reference max and sum [unit][128 queries], unit = workgroup
+  // Query blocks of all heads, in order: the first `whole` walk all their keys, one workgroup each; the `tail` after
+  // them have `splits` workgroups each, which take a contiguous range of the tiles.
+  int whole, tail, splits;
+  float4* po;             // the tail's unnormalized partial outputs [split][tail block][32 chunks of 4 dims][128 queries]
+  float2* pml;            // and their reference max and sum [split][tail block][128 queries]
   int ngroups;
   AttnGroup group[kMaxGroups];
 };
@@ -112,9 +114,12 @@ void attention_kernel(const AttnArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h2 = lane >> 5, l32 = lane & 31;
-  // the workgroups of one (batch, head) and key range run side by side, so their tiles are read once from HBM
-  const int range = blockIdx.x / a.qblocks, qb = blockIdx.x % a.qblocks;
-  const int bh = SPLIT ? range / a.splits : range, split = SPLIT ? range % a.splits : 0;
+  // (query blocks of one head run side by side, so that their tiles are read once from HBM)
+  const bool part = SPLIT && (int)blockIdx.x >= a.whole;
+  const int slot = part ? blockIdx.x - a.whole : 0;  // of the partials
+  const int split = part ? slot / a.tail : 0;
+  const int unit = part ? a.whole + slot % a.tail : blockIdx.x;
+  const int bh = unit / a.qblocks, qb = unit % a.qblocks;
   const int64_t b = bh / a.H, hh = bh % a.H;
   int gi = 0;
   while (gi + 1 < a.ngroups && qb >= a.group[gi + 1].qb0) gi++;
@@ -217,7 +222,7 @@ void attention_kernel(const AttnArgs a) {
   int nt = (t_n + kBK - 1) / kBK;  // tiles of all segments
   for (int i = 0; i < a.nseg; i++) nt += (int)((a.seg[i].len + kBK - 1) / kBK);
   next_segment();
-  if constexpr (SPLIT) {  // this workgroup's tiles [skip, skip + nt)
+  if (part) {  // this workgroup's tiles [skip, skip + nt)
     int skip = (int)((int64_t)nt * split / a.splits);
     nt = (int)((int64_t)nt * (split + 1) / a.splits) - skip;
     for (int64_t here; (here = (left + kBK - 1) / kBK) <= skip;) {
@@ -350,15 +355,15 @@ void attention_kernel(const AttnArgs a) {
   for (int i = 0; i < 32; i++) lsum += pv[i];
   // normalize and store: lane holds query l32, dims 32 db + 8 rr + 4 h2 + 0..3 in registers 4 rr .. 4 rr + 3
   const float ltot = lsum + __shfl_xor(lsum, 32);
-  if constexpr (SPLIT) {  // fp32 partials, 16 bytes per lane with the 32 queries side by side
-    float4* po = a.po + (int64_t)blockIdx.x * 32 * kBQ + wave * 32 + l32;
+  if (part) {  // fp32 partials, 16 bytes per lane with the 32 queries side by side
+    float4* po = a.po + (int64_t)slot * 32 * kBQ + wave * 32 + l32;
 #pragma unroll
     for (int db = 0; db < 4; db++)
 #pragma unroll
       for (int rr = 0; rr < 4; rr++)
         po[(8 * db + 2 * rr + h2) * kBQ] =
             make_float4(oacc[db][4 * rr], oacc[db][4 * rr + 1], oacc[db][4 * rr + 2], oacc[db][4 * rr + 3]);
-    if (h2 == 0) a.pml[(int64_t)blockIdx.x * kBQ + wave * 32 + l32] = make_float2(m, ltot);
+    if (h2 == 0) a.pml[(int64_t)slot * kBQ + wave * 32 + l32] = make_float2(m, ltot);
     return;
   }
   const float inv = 1.0f / ltot;
@@ -383,7 +388,7 @@ constexpr int kCombineThreads = 256;
 
 __global__ __launch_bounds__(kCombineThreads) void attention_combine_kernel(const AttnArgs a) {
   const int ql = (blockIdx.x % 4) * 32 + (threadIdx.x & 31), part = threadIdx.x >> 5;
-  const int unit = blockIdx.x / 4;
+  const int unit = a.whole + blockIdx.x / 4;
   const int bh = unit / a.qblocks, qb = unit % a.qblocks;
   int gi = 0;
   while (gi + 1 < a.ngroups && qb >= a.group[gi + 1].qb0) gi++;
@@ -391,14 +396,14 @@ __global__ __launch_bounds__(kCombineThreads) void attention_combine_kernel(cons
   if (qi >= a.group[gi].q_n) return;
   const int64_t qrow = a.rows ? a.rows[a.group[gi].q_off + qi] : qi;
   if (a.owner != nullptr && a.owner[qrow] != gi) return;
-  const int64_t first = (int64_t)bh * a.splits * a.qblocks + qb;  // the unit's workgroup of split s: first + s qblocks
+  const int64_t first = blockIdx.x / 4;  // the block's partial of split s: first + s tail
   float mmax = -__builtin_inff();
-  for (int s = 0; s < a.splits; s++) mmax = __builtin_fmaxf(mmax, a.pml[(first + (int64_t)s * a.qblocks) * kBQ + ql].x);
+  for (int s = 0; s < a.splits; s++) mmax = __builtin_fmaxf(mmax, a.pml[(first + (int64_t)s * a.tail) * kBQ + ql].x);
   float o[16], l = 0.0f;
 #pragma unroll
   for (int i = 0; i < 16; i++) o[i] = 0.0f;
   for (int s = 0; s < a.splits; s++) {
-    const int64_t wg = first + (int64_t)s * a.qblocks;
+    const int64_t wg = first + (int64_t)s * a.tail;
     const float2 ml = a.pml[wg * kBQ + ql];
     const float w = __builtin_amdgcn_exp2f(ml.x - mmax);
     l = __builtin_fmaf(w, ml.y, l);
@@ -529,61 +534,72 @@ __global__ __launch_bounds__(kPackThreads) void attention_pack_kernel(const Pack
 
 int64_t tiles_of(int64_t n) { return (n + kBK - 1) / kBK; }
 
-// How many workgroups share one query block's keys, from the number of query blocks (units) and their key tiles.
-// Times are in tiles of a compute unit that holds two workgroups: a round of workgroups takes its tiles plus about
-// four for its start and end, a last round of at most one workgroup per unit 0.7 of that (its waves have the SIMD
-// to themselves), a combine pass its launch and 128 KB of traffic per workgroup.  Ranges stay at four tiles or
-// more, workgroups at four rounds (the partials' memory), and a split has to promise a twentieth.  Measured whole
-// calls, one range against the chosen number: 16 units x 290 tiles 316 -> 61 us, 40 x 73 89 -> 40, 144 x 49 69 -> 58,
-// 216 x 129 191 -> 148, 336 x 182 330 -> 281, 592 x 213 618 -> 527; from about two rounds of units up the best
-// number gains under 2 % and one range stays.  The choice lies within 5 % of the best of 1 to 32 throughout.
-int choose_splits(int64_t units, int64_t tiles) {
+// How the query blocks (units) of a call share their key tiles: the first `whole` take one workgroup each, the others
+// `splits`.  Times are in tiles of a compute unit that holds two workgroups: a round of workgroups takes its tiles plus
+// about four for its start and end, a last round of at most one workgroup per unit 0.7 of that (its waves have the SIMD
+// to themselves), a combine pass its launch and 128 KB of traffic per workgroup.  Whole rounds stay whole (their partials
+// would be traffic for nothing), or nothing does; ranges stay at four tiles or more, split workgroups at four rounds (the
+// partials' memory), and a split has to promise a thirtieth, of a
+// last round alone a sixtieth.
+// Measured whole calls, no split against the chosen one (us): 16 units x 290 tiles 316 -> 61, 40 x 73 89 -> 40, 144 x 49
+// 69 -> 58, 216 x 129 191 -> 148, 336 x 182 330 -> 281, 592 x 213 618 -> 506; with a split last round only, 1024 x 157
+// 760 -> 665, 1560 x 129 853 -> 790, 3168 x 264 3165 -> 3038, 3344 x 416 5330 -> 5090.
+struct Split {
+  int64_t whole;
+  int splits;
+};
+Split choose_splits(int64_t units, int64_t tiles) {
   const int64_t cus = cu_count(), slots = 2 * cus;
-  auto cost = [&](int64_t s) {
-    const int64_t full = units * s / slots, rem = units * s % slots;
+  auto cost = [&](int64_t whole, int64_t s) {
+    const int64_t wgs = (units - whole) * s, full = wgs / slots, rem = wgs % slots;
     const double rounds = full + (rem == 0 ? 0.0 : rem <= cus ? 0.7 : 1.0);
-    return rounds * ((tiles + s - 1) / s + 4) + (s > 1 ? 2.0 + 0.016 * units * s : 0.0);
+    return (double)(whole / slots) * (tiles + 4) + rounds * ((tiles + s - 1) / s + 4) + (s > 1 ? 2.0 + 0.016 * wgs : 0.0);
   };
-  int best = 1;
-  double least = 0.95 * cost(1);
-  for (int64_t s = 2; s <= 64 && s * 4 <= tiles && units * s <= 4 * slots; s++)
-    if (cost(s) < least) {
-      best = (int)s;
-      least = cost(s);
-    }
+  Split best{0, 1};
+  const double one = cost(0, 1);
+  double least = one;
+  const int64_t rounds = units / slots * slots;
+  for (int64_t whole : {(int64_t)0, rounds})
+    for (int64_t s = 2; s <= 64 && s * 4 <= tiles && (units - whole) * s <= 4 * slots && units > whole; s++)
+      if (cost(whole, s) < least && cost(whole, s) < one * (whole ? 59.0 / 60 : 29.0 / 30)) {
+        best = Split{whole, (int)s};
+        least = cost(whole, s);
+      }
   return best;
 }
 
-// Bytes of the partials of `units` query blocks in `splits` ranges: outputs, then maxima and sums.
-int64_t partial_bytes(int64_t units, int splits) {
-  return splits > 1 ? units * splits * kBQ * (kHeadDim * 4 + 8) : 0;
+// Bytes of the partials of `units` query blocks: outputs, then maxima and sums.
+int64_t partial_bytes(int64_t units, Split sp) {
+  return sp.splits > 1 ? (units - sp.whole) * sp.splits * kBQ * (kHeadDim * 4 + 8) : 0;
 }
 
 // Launches the attention kernel over args whose pointers, strides, segments and groups are set; `partials` is
-// where the partials of `splits` > 1 go.
-int launch_attention(AttnArgs& a, int64_t B, float scale, int splits, char* partials, hipStream_t st) {
+// where the partials of split blocks go.
+int launch_attention(AttnArgs& a, int64_t B, float scale, Split sp, char* partials, hipStream_t st) {
   int64_t qblocks = 0;
   for (int g = 0; g < a.ngroups; g++) {
     a.group[g].qb0 = (int)qblocks;
     qblocks += ((int64_t)a.group[g].q_n + kBQ - 1) / kBQ;
   }
   const int64_t units = B * a.H * qblocks;
-  HN_REQUIRE(units * splits <= 0x7fffffff, "hn_attention: problem too large");
+  HN_REQUIRE(units * sp.splits <= 0x7fffffff, "hn_attention: problem too large");
   if (units == 0) return HN_OK;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.qblocks = (int)qblocks;
-  a.splits = splits;
-  const dim3 grid((unsigned)(units * splits)), block(kAttnWaves * 64);
-  if (splits == 1) {
+  a.splits = sp.splits;
+  a.whole = (int)sp.whole;
+  a.tail = (int)(units - sp.whole);
+  const dim3 grid((unsigned)(sp.splits > 1 ? sp.whole + a.tail * (int64_t)sp.splits : units)), block(kAttnWaves * 64);
+  if (sp.splits == 1) {
     hipLaunchKernelGGL(attention_kernel<false>, grid, block, 0, st, a);
     return HN_LAUNCH_CHECK("attention_kernel");
   }
   a.po = (float4*)partials;
-  a.pml = (float2*)(partials + units * splits * kBQ * kHeadDim * 4);
+  a.pml = (float2*)(partials + (int64_t)a.tail * sp.splits * kBQ * kHeadDim * 4);
   hipLaunchKernelGGL(attention_kernel<true>, grid, block, 0, st, a);
   const int rc = HN_LAUNCH_CHECK("attention_kernel");
   if (rc != HN_OK) return rc;
-  hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)(units * 4)), dim3(kCombineThreads), 0, st, a);
+  hipLaunchKernelGGL(attention_combine_kernel, dim3((unsigned)a.tail * 4), dim3(kCombineThreads), 0, st, a);
   return HN_LAUNCH_CHECK("attention_combine_kernel");
 }
 
@@ -591,7 +607,7 @@ int launch_attention(AttnArgs& a, int64_t B, float scale, int splits, char* part
 // owner of each query row, the partials of split keys; each from a 256-byte boundary.
 struct SegmentLayout {
   int64_t positions, t_rows, tk, owner, partials, bytes;
-  int splits;
+  Split split;
 };
 SegmentLayout segment_layout(const int64_t* parts, int n_parts, const int64_t* groups, int n_groups, int64_t B,
                              int64_t H, int64_t Lq) {
@@ -607,12 +623,12 @@ SegmentLayout segment_layout(const int64_t* parts, int n_parts, const int64_t* g
   for (int p = 0; p < n_parts; p++) tiles += tiles_of(parts[9 * p + 8]);
   l.positions = l.t_rows + tiles * kBK;
   const int64_t units = B * H * qblocks;
-  l.splits = choose_splits(units, tiles + (fewest > 0 ? fewest : 0));  // every group has a tile for every range
+  l.split = choose_splits(units, tiles + (fewest > 0 ? fewest : 0));  // every group has a tile for every range
   auto align = [](int64_t x) { return (x + 255) / 256 * 256; };
   l.tk = align(B * H * kHeadDim * l.positions * 2);
   l.owner = l.tk + align(B * H * kHeadDim * l.t_rows * 2);
   l.partials = l.owner + (n_groups ? align(Lq * 4) : 0);
-  l.bytes = l.partials + partial_bytes(units, l.splits);
+  l.bytes = l.partials + partial_bytes(units, l.split);
   return l;
 }
 
@@ -653,11 +669,11 @@ static int attention_impl(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, 
   a.ngroups = 1;
   a.group[0] = AttnGroup{0, 0, (int)Lq, 0, 0};
   const int64_t units = B * H * ((Lq + kBQ - 1) / kBQ);
-  const int splits = workspace ? choose_splits(units, tiles_of(Lk)) : 1;
-  HN_REQUIRE(workspace_bytes >= partial_bytes(units, splits) && ((uintptr_t)workspace & 15) == 0,
+  const Split split = workspace ? choose_splits(units, tiles_of(Lk)) : Split{0, 1};
+  HN_REQUIRE(workspace_bytes >= partial_bytes(units, split) && ((uintptr_t)workspace & 15) == 0,
              "hn_attention_ws: workspace of %lld bytes (16-byte aligned), %lld needed", (long long)workspace_bytes,
-             (long long)partial_bytes(units, splits));
-  return launch_attention(a, B, scale, splits, (char*)workspace, (hipStream_t)stream);
+             (long long)partial_bytes(units, split));
+  return launch_attention(a, B, scale, split, (char*)workspace, (hipStream_t)stream);
 }
 
 extern "C" int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb,
@@ -777,5 +793,5 @@ extern "C" int hn_segment_attention(const void* q, int64_t sqb, int64_t sqh, int
   const dim3 grid((unsigned)(p.tiles + (n_groups ? 1 : 0)), (unsigned)(B * H));
   hipLaunchKernelGGL(attention_pack_kernel, grid, dim3(kPackThreads), 0, (hipStream_t)stream, p);
   const int rc = HN_LAUNCH_CHECK("attention_pack_kernel");
-  return rc != HN_OK ? rc : launch_attention(a, B, scale, l.splits, ws + l.partials, (hipStream_t)stream);
+  return rc != HN_OK ? rc : launch_attention(a, B, scale, l.split, ws + l.partials, (hipStream_t)stream);
 }

@@ -46,7 +46,9 @@ def per_group(q, k, v, hist, plan):
     # few queries over many keys: several workgroups share a query block's keys, with ranges that start and end in
     # the history, the video keys and the text keys
     (1, 2, 129, 40, 1900, 3, False), (2, 1, 40, 200, 511, 2, True), (1, 1, 900, 1, 0, 1, False),
-    (1, 3, 20, 600, 64, 1, False)])
+    (1, 3, 20, 600, 64, 1, False),
+    # more query blocks than a round of workgroups (512 on 256 compute units): only those past it are split
+    (1, 24, 2700, 100, 300, 2, False), (2, 20, 1700, 3, 0, 1, True)])
 def test_groups_against_float32(dev, b, h, lv, lt, lh, n, head_major):
     from hy_nomas import attention
 
