@@ -14,16 +14,20 @@ constexpr int64_t kWholeKInt32Limit = 131072;
 // The rows of a problem, as two launches: a.M rows from row 0 with the big tile, then the rest with a 128 x 128
 // tile.  Tile rows are independent and every output keeps its fold order, so the results do not depend on
 // where the split falls.
-enum class TileSplit { kBig, kSmall, kBoth };
+enum class TileSplit { kBig, kMid, kSmall, kBoth };
 
 // Which tiles serve an M x N problem whose big tile is bm x bn with `slots` workgroups resident (one round of
 // tiles), and for kBoth the rows the big tile takes.  A persistent grid runs ceil(tiles / slots) rounds of
 // tiles; when the last round would leave more than half of the compute units idle, its rows go to 128 x 128
 // tiles (four per big tile, on every compute unit).  A problem with fewer big tiles than half a round runs on
-// small tiles alone.
+// small tiles alone, and one whose bn x 192 tiles still fit one round takes those: the round is shorter (256 x 192
+// against 256 x 256 tiles, us, g128 / per token / fp8 blocks: 3520 x 12288 -> 3072 218 / 146 / 163 -> 191 / 135 / 148,
+// 3520 x 3072 -> 3072 64.8 / 39.7 / 48.8 -> 55.6 / 34.4 / 41.3, 5000 x 8192 -> 2048 143 / 96 / 107 -> 128 / 90 / 99).  With
+// more rounds than one they lose what they gain: a round of them takes 0.9 of the big tile's for 0.75 of its work.
 static TileSplit choose_tiles(int64_t M, int64_t N, int bm, int bn, int64_t slots, int64_t* big_rows) {
   const int64_t tm = (M + bm - 1) / bm, tn = (N + bn - 1) / bn, tiles = tm * tn;
   const int64_t full = tiles / slots, rem = tiles % slots;
+  if (full == 0 && rem > slots / 2 && (M + 191) / 192 * tn <= slots) return TileSplit::kMid;
   if (rem == 0 || rem > slots / 2) return TileSplit::kBig;
   if (full == 0) return TileSplit::kSmall;
   const int64_t rows = (full * slots / tn) * bm;  // whole tile rows of the full rounds
@@ -32,14 +36,15 @@ static TileSplit choose_tiles(int64_t M, int64_t N, int bm, int bn, int64_t slot
   return TileSplit::kBoth;
 }
 
-// Launch the big-tile configuration BIG or the small one SMALL (each a launch_cfg instantiation) over the rows
-// choose_tiles assigns them.
-template <int BM, int BN, int WN, int WM, int WPE, typename Big, typename Small>
-static int launch_split(GemmArgs& a, int out_esz, hipStream_t st, Big big, Small small) {
+// Launch the tile configurations BIG, MID and SMALL (each a launch_cfg instantiation) over the rows choose_tiles
+// assigns them.
+template <int BM, int BN, int WN, int WM, int WPE, typename Big, typename Mid, typename Small>
+static int launch_split(GemmArgs& a, int out_esz, hipStream_t st, Big big, Mid mid, Small small) {
   const int64_t slots = (int64_t)cu_count() * (WPE * 4 / (WN * WM));
   int64_t rows = 0;
   const TileSplit how = choose_tiles(a.M, a.N, BM, BN, slots, &rows);
   if (how == TileSplit::kBig) return big(a);
+  if (how == TileSplit::kMid) return mid(a);
   if (how == TileSplit::kSmall) return small(a);
   GemmArgs head = a, tail = a;
   head.M = rows;
@@ -54,7 +59,8 @@ static int launch_split(GemmArgs& a, int out_esz, hipStream_t st, Big big, Small
 // per-token / per-channel: 256 x 256 tile, 8 waves of 128 x 64.  fp8 with block weight scales: the same
 // tile (the running sum is rescaled in place, so there is no second accumulator set).  Other g128 layouts:
 // 256 x 128, 8 waves of 128 x 32 (the int32 group partial and the fp32 running sum both fit in 256
-// VGPRs).  128-byte K stages in two LDS buffers.  The plain and GELU epilogues also have 128 x 128 tiles of
+// VGPRs).  128-byte K stages in two LDS buffers.  The plain and GELU epilogues also have tiles of 256 channels x 192
+// tokens (eight waves of 64 x 96) and of 128 x 128 in
 // four waves (64 x 64 each, or 128 x 32 with block weight scales) for problems, or tails of problems, that
 // would leave most compute units idle with the big tile (choose_tiles); two such workgroups share a compute
 // unit (about 70 KB of LDS each).
@@ -70,8 +76,9 @@ static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
   if (!g128) {
     auto big = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, false, 2, 4, 4, 2, OUT_DT, 128, 2>(x, st); };
     if constexpr (SMALL_OK) {
+      auto mid = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, false, 4, 2, 2, 3, OUT_DT, 128, 2>(x, st); };
       auto small = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, false, 2, 2, 2, 2, OUT_DT, 128, 2, false, 2>(x, st); };
-      return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, small);
+      return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, mid, small);
     }
     if constexpr (WAVE_ROWS)
       if (int64_t rows = 0; choose_tiles(a.M, a.N, 256, 256, cu_count(), &rows) == TileSplit::kSmall)
@@ -82,10 +89,11 @@ static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
     if (a.sw_rows == 128) {
       auto big = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, true, 2, 4, 4, 2, OUT_DT, 128, 2, true>(x, st); };
       if constexpr (SMALL_OK) {
+        auto mid = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, true, 4, 2, 2, 3, OUT_DT, 128, 2, true>(x, st); };
         auto small = [&](GemmArgs& x) {
           return launch_cfg<KIND, EPI, true, 1, 4, 4, 1, OUT_DT, 128, 2, true, 2>(x, st);
         };
-        return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, small);
+        return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, mid, small);
       }
       return big(a);
     }
@@ -96,8 +104,9 @@ static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
     }
     auto big = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, true, 2, 4, 4, 2, OUT_DT, 128, 2>(x, st); };
     if constexpr (SMALL_OK) {
+      auto mid = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, true, 4, 2, 2, 3, OUT_DT, 128, 2>(x, st); };
       auto small = [&](GemmArgs& x) { return launch_cfg<KIND, EPI, true, 2, 2, 2, 2, OUT_DT, 128, 2, false, 2>(x, st); };
-      return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, small);
+      return launch_split<256, 256, 2, 4, 2>(a, ESZ, st, big, mid, small);
     }
     if constexpr (WAVE_ROWS)
       if (int64_t rows = 0; choose_tiles(a.M, a.N, 256, 256, cu_count(), &rows) == TileSplit::kSmall)

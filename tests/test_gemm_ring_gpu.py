@@ -72,3 +72,32 @@ def test_four_wave_tiles_of_the_fused_epilogues(dev, per_channel, m, n, k):
         # one bf16 rounding of the normalized value may fall the other way (2^-8), and its product's with it
         assert ((hm[part] - want).float().abs() <= want.float().abs() * 2 ** -6 + 1e-6).all()
         assert (hm[part] != want).float().mean() < 1e-2
+
+
+@pytest.mark.parametrize("m,n,k", [(3400, 2816, 128), (3265, 2700, 384), (3072, 3000, 640), (300, 24576, 256)])
+@pytest.mark.parametrize("layout", ["g128", "channel", "fp8"])
+def test_mid_tile_rows_equal_the_small_tiles(dev, layout, m, n, k):
+    """Problems of one round of 256 x 192 tiles (129 to 192 tiles of 256 x 256 on 256 compute units), cut by M and N:
+    rows of every part of a tile equal the same rows run alone, which take other tiles, bit for bit."""
+    from hy_nomas import kernels
+
+    print(f"mid tile {layout} m={m} n={n} k={k}", flush=True)
+    g = seeded(m + n + k)
+    kind = "fp8" if layout == "fp8" else "int8"
+    qa, sa = kernels.quantize_activations(outlier_input(m, k, seed=m).to(dev), kind, None if layout == "channel" else 128)
+    if kind == "fp8":
+        w = (torch.randn(n, k, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)
+        sw = torch.rand((n + 127) // 128, k // 128, generator=g) * 4e-3 + 1e-3
+        bias = (torch.randn(n, generator=g) * 0.02).to(torch.bfloat16)
+    else:
+        w, sw, bias = int8_weights(n, k, n + 3 * k, per_channel=layout == "channel")
+    w, sw, bias = w.to(dev), sw.to(dev), bias.to(dev)
+    kernels.validate_scales(sw)
+    rows = torch.cat([torch.arange(0, 16), torch.arange(88, 104), torch.arange(184, 200), torch.arange(m - 20, m)]).to(dev)
+    sa_rows = sa[rows].contiguous()
+    kernels.validate_scales(sa_rows)
+    for dt in (torch.bfloat16, torch.float32):
+        for epi in (None, "gelu"):
+            full = kernels.block_gemm(qa, sa, w, sw, bias, dt, kind, epi)
+            part = kernels.block_gemm(qa[rows].contiguous(), sa_rows, w, sw, bias, dt, kind, epi)
+            assert torch.equal(full[rows], part), (dt, epi)
