@@ -136,7 +136,7 @@ def _tiled(n):
 def _attend_parts(q, parts, out=None):
     """Attention of every query to the keys of all (k, v) `parts`, read where they lie."""
     q = _rows16(q)
-    parts = [(_rows16(k), _rows16(v)) for k, v in parts]
+    parts = [(_rows16(k), _rows16(v), k.shape[1]) for k, v in parts]
     if out is None:
         out = torch.empty(q.shape, device=q.device, dtype=torch.bfloat16)
     _segment_call(q, parts, None, [], None, 0, out)
@@ -144,8 +144,9 @@ def _attend_parts(q, parts, out=None):
 
 
 def _segment_call(q, parts, text, groups, rows, text_off, out):
+    """One `hn_segment_attention` call; parts (k, v, n): the first n keys of k and v."""
     b, lq, h, d = q.shape
-    pt = _lib.int64s([x for k, v in parts for x in (*_operand(k), *_operand(v), k.shape[1])])
+    pt = _lib.int64s([x for k, v, n in parts for x in (*_operand(k), *_operand(v), n)])
     tx = _lib.int64s([*_operand(text[0]), *_operand(text[1])]) if text is not None else None
     gr = _lib.int64s([x for g in groups for x in g]) if groups else None
     nbytes = _lib.lib().hn_segment_attention_workspace_bytes(pt, len(parts), gr, len(groups), b, h, lq)
@@ -175,8 +176,8 @@ def _attend_groups(q, k, v, hist, plan, out):
     each group's text keys gathered.  A row that several groups name takes the last one's result."""
     lv, length = plan.video_tokens, q.shape[1]
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
-    parts = [(_rows16(hist[0]), _rows16(hist[1]))] if hist is not None and hist[0].shape[1] else []
-    parts.append((k[:, :lv], v[:, :lv]))
+    parts = [(_rows16(hist[0]), _rows16(hist[1]), hist[0].shape[1])] if hist is not None and hist[0].shape[1] else []
+    parts.append((k, v, lv))
     for first in range(0, len(plan.groups), MAX_GROUPS):
         chunk = plan.groups[first:first + MAX_GROUPS]
         idx = torch.cat([t for t, _ in chunk] + [t for _, t in chunk])

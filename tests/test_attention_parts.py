@@ -42,7 +42,7 @@ def per_group(q, k, v, hist, plan):
 @pytest.mark.parametrize("b,h,lv,lt,lh,n,head_major", [
     (1, 2, 63, 7, 0, 2, False), (1, 3, 64, 64, 64, 1, False), (2, 2, 129, 5, 65, 3, False), (1, 1, 1, 1, 1, 1, True),
     (2, 3, 300, 130, 191, 4, True), (1, 2, 200, 3, 127, 5, False), (1, 2, 130, 0, 70, 2, False),
-    (1, 1, 150, 70, 33, 70, False),
+    (1, 1, 150, 70, 33, 70, False), (1, 2, 0, 40, 0, 2, False), (1, 2, 0, 33, 70, 2, False),
     # few queries over many keys: several workgroups share a query block's keys, with ranges that start and end in
     # the history, the video keys and the text keys
     (1, 2, 129, 40, 1900, 3, False), (2, 1, 40, 200, 511, 2, True), (1, 1, 900, 1, 0, 1, False),
