@@ -59,11 +59,10 @@ static int launch_split(GemmArgs& a, int out_esz, hipStream_t st, Big big, Mid m
 // per-token / per-channel: 256 x 256 tile, 8 waves of 128 x 64.  fp8 with block weight scales: the same
 // tile (the running sum is rescaled in place, so there is no second accumulator set).  Other g128 layouts:
 // 256 x 128, 8 waves of 128 x 32 (the int32 group partial and the fp32 running sum both fit in 256
-// VGPRs).  128-byte K stages in two LDS buffers.  The plain and GELU epilogues also have tiles of 256 channels x 192
-// tokens (eight waves of 64 x 96) and of 128 x 128 in
-// four waves (64 x 64 each, or 128 x 32 with block weight scales) for problems, or tails of problems, that
-// would leave most compute units idle with the big tile (choose_tiles); two such workgroups share a compute
-// unit (about 70 KB of LDS each).
+// VGPRs).  128-byte K stages in two LDS buffers.  The plain and GELU epilogues also have tiles for problems, or
+// tails of problems, that would leave many compute units idle with the big tile (choose_tiles): 256 channels x 192
+// tokens in eight waves of 64 x 96, and 128 x 128 in four waves (64 x 64 each, or 128 x 32 with block weight scales), of
+// which two workgroups share a compute unit (about 70 KB of LDS each).
 template <int KIND, int EPI, int OUT_DT>
 static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
   constexpr bool SWIGLU = EPI == HN_EPI_SWIGLU_QUANT;
@@ -203,7 +202,7 @@ static int launch_skinny_x_dt(GemmArgs& a, bool g128, int rounding, hipStream_t 
 }
 
 // Up to four rows whose codes fit 48 KB of LDS (three workgroups on a compute unit), 16-byte aligned, in a quantization
-// that the quantizer takes.  3072 -> 18432 at one row: quantizer and GEMM 2.6 + 11.5 us.
+// that the quantizer takes.  3072 -> 18432 at one row: 12.9 us, against 2.6 + 11.5 us for quantizer and GEMM.
 bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t group, int kind,
                          int rounding, int out_dtype) {
   return M > 0 && M <= kSkinnyMaxM && kind == HN_KIND_INT8 && (x_dtype == HN_DTYPE_BF16 || x_dtype == HN_DTYPE_F16) &&
