@@ -102,7 +102,7 @@ int hn_block_gemm(const void* qa, int64_t lda, const float* sa, int64_t ldsa, co
  *   K: one scale per token) with `kind` codes and `rounding`; the codes and scales are written to
  *   `workspace` (256-byte aligned, at least hn_block_linear_workspace_bytes(M, K, group) bytes; its contents
  *   on entry do not matter and are overwritten) and multiplied with qw / sw / bias as hn_block_gemm does,
- *   into out [M, N] of out_dtype (row stride ldo).
+ *   into out [M, N] of out_dtype (row stride ldo).  out may lie in x's memory: x is read whole first.
  * With kind FP8 and sw_rows == 128 the weight scales must be positive and finite.
  */
 int64_t hn_block_linear_workspace_bytes(int64_t M, int64_t K, int64_t group);

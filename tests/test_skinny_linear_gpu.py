@@ -35,3 +35,45 @@ def test_equals_quantizer_then_gemm(dev, layout, m, n, k):
             wide = torch.zeros(m, k + 64, dtype=dt, device=dev)
             wide[:, :k] = xd
             assert torch.equal(kernels.block_linear(wide[:, :k], w.to(dev), sw.to(dev), b, rounding=rounding), want)
+
+
+def entry(x, ldx, m, n, k, group, w, sw, sw_rows, bias, out, ldo, ws, rounding="half_away"):
+    """hn_block_linear on the caller's own buffers."""
+    from hy_nomas import _lib
+
+    _lib.call("hn_block_linear", x.data_ptr(), _lib.dtype_code(x), ldx, m, k, group, 0, _lib.ROUND[rounding], w.data_ptr(), k,
+              sw.data_ptr(), sw.stride(0), sw_rows, bias.data_ptr(), _lib.dtype_code(bias), n, out.data_ptr(),
+              _lib.dtype_code(out), ldo, ws.data_ptr(), ws.numel(), _lib.stream(x))
+
+
+def linear_case(dev, layout, m, n, k, dt=torch.bfloat16):
+    w, sw, bias = int8_weights(n, k, n + k, layout == "channel")
+    if layout == "block":
+        sw = sw[:: 128].contiguous()
+    x = torch.randn(m, k, generator=seeded(m + k)).to(dt).to(dev)
+    return (x, w.to(dev), sw.to(dev), bias.to(dt).to(dev), k if layout == "channel" else 128,
+            128 if layout == "block" else 1)
+
+
+@pytest.mark.parametrize("layout", ["g128", "channel"])
+@pytest.mark.parametrize("m,n,k,at", [(1, 3072, 3072, 0), (4, 3072, 3072, 0), (4, 12288, 12288, 0), (2, 1000, 1152, 576),
+                                      (3, 6000, 8192, -64)])
+def test_output_over_the_source(dev, layout, m, n, k, at):
+    """out in x's own rows, from column `at` on (before the first row: at < 0): every value of x is read before any output
+    is stored, as with more rows, by either entry point."""
+    from hy_nomas import _lib, kernels
+    from test_zz_no_alloc import noalloc
+
+    x, w, sw, bias, group, sw_rows = linear_case(dev, layout, m, n, k)
+    want = kernels.block_linear(x, w, sw, bias)
+    ld = max(k, n) + 64
+    ws = torch.empty(_lib.lib().hn_block_linear_workspace_bytes(m, k, group), device=dev, dtype=torch.uint8)
+    for held in (True, False):
+        buf = torch.zeros(64 + (m + 1) * ld, dtype=x.dtype, device=dev)
+        src, out = buf[64:].as_strided((m, k), (ld, 1)), buf[64 + at:].as_strided((m, n), (ld, 1))
+        src.copy_(x)
+        if held:
+            entry(src, ld, m, n, k, group, w, sw, sw_rows, bias, out, ld, ws)
+        else:
+            noalloc(src, w, sw, bias, group, "int8", out=out)
+        assert torch.equal(out, want)
