@@ -210,7 +210,7 @@ bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int
          ((uintptr_t)x & 15) == 0 && (rounding == HN_ROUND_HALF_AWAY || rounding == HN_ROUND_HALF_EVEN);
 }
 
-// hn_block_gemm, or (x given, skinny_takes_source) the linear of x itself; qa and sa are then not read.
+// hn_block_gemm, or (x given, skinny_takes_source) the linear of x itself; qa [M, K] and sa [M, K / group] are then written.
 static int block_gemm_impl(const void* x, int64_t ldx, int rounding, const void* qa, int64_t lda, const float* sa,
                            int64_t ldsa, const void* qw, int64_t ldw, const float* sw, int64_t ldsw, int64_t sw_rows,
                            const void* bias, int bias_dtype, int64_t M, int64_t N, int64_t K, int64_t group, int kind,

@@ -25,23 +25,24 @@ int check_linear(const char* who, const void* x, int64_t M, int64_t N, int64_t K
   return HN_OK;
 }
 
-// Whether M rows of K values at x and M rows of N values at out (2 bytes each) share a byte, gaps between rows counted in.
-static bool rows_overlap(const void* x, int64_t ldx, int64_t K, const void* out, int64_t ldo, int64_t N, int64_t M) {
-  const uintptr_t xb = (uintptr_t)x, ob = (uintptr_t)out;
-  return xb < ob + 2 * ((M - 1) * ldo + N) && ob < xb + 2 * ((M - 1) * ldx + K);
+// Whether the np bytes at p and the nq bytes at q share one.
+static bool overlap(const void* p, int64_t np, const void* q, int64_t nq) {
+  return (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
 }
 
 // Quantize x into the workspace, then run the GEMM from it (both enqueued on `stream`); a few rows of 16-bit x go to the
-// skinny kernel, which quantizes them itself (gemm.hip).  Its workgroups read x while others store their outputs, so an
-// output in x's own memory keeps the two passes: x is read whole before anything is stored.
+// skinny kernel, which quantizes them itself (gemm.hip) and leaves the codes and scales in the workspace too.  Its
+// workgroups read x while others store, so an output or a workspace in x's own memory (the gaps between rows counted in)
+// keeps the two passes: x is read whole before an output is stored.
 int run_linear(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t group, int kind, int rounding,
                const void* qw, int64_t ldw, const float* sw, int64_t ldsw, int64_t sw_rows, const void* bias,
                int bias_dtype, int64_t N, void* out, int out_dtype, int64_t ldo, uint8_t* ws, void* stream) {
   if (M == 0) return HN_OK;
   float* s = reinterpret_cast<float*>(ws + linear_scales_offset(M, K));
   const int64_t ng = K / group;
+  const int64_t x_bytes = 2 * ((M - 1) * ldx + K);
   if (skinny_takes_source(x, x_dtype, ldx, M, K, group, kind, rounding, out_dtype) &&
-      !rows_overlap(x, ldx, K, out, ldo, N, M))
+      !overlap(x, x_bytes, out, 2 * ((M - 1) * ldo + N)) && !overlap(x, x_bytes, ws, linear_workspace_bytes(M, K, group)))
     return skinny_linear(x, ldx, rounding, ws, s, qw, ldw, sw, ldsw, sw_rows, bias, bias_dtype, M, N, K, group, out, out_dtype,
                          ldo, stream);
   int rc = hn_quantize_act(x, x_dtype, ldx, M, K, group, kind, rounding, ws, K, s, ng, stream);

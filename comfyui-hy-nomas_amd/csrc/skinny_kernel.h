@@ -13,7 +13,8 @@
 //
 // With a source (SRC, the linear's 16-bit x) the kernel quantizes it itself: each workgroup forms the codes and scales
 // of its M rows in LDS, with the quantizer's own arithmetic, while its first weights are on the way.  At most 48 KB
-// of codes, read from L2 by every workgroup; in return the quantizer's launch and the codes' trip through memory go.
+// of codes, read from L2 by every workgroup; in return the quantizer's launch and the codes' trip through memory go.  The
+// first workgroup also leaves them in a.qa and a.sa, the workspace where the linear's callers find them.
 #pragma once
 
 #include "gemm_kernel.h"
@@ -30,6 +31,15 @@ constexpr int kSkinnyMaxM = 4;
 template <bool PER_TOKEN, int DT, int ROUND>
 __device__ __forceinline__ void quantize_rows(const GemmArgs& a, uint8_t* codes, float* scales) {
   constexpr int T = kSkinnyWaves * 64;
+  const bool keep = blockIdx.x == 0;
+  auto put = [&](int at, uint2 c) __attribute__((always_inline)) {  // 8 codes from flat position `at` on
+    *reinterpret_cast<uint2*>(codes + at) = c;
+    if (keep) *reinterpret_cast<uint2*>(const_cast<uint8_t*>(a.qa) + at) = c;
+  };
+  auto put_scale = [&](int at, float sc) __attribute__((always_inline)) {
+    scales[at] = sc;
+    if (keep) const_cast<float*>(a.sa)[at] = sc;
+  };
   __shared__ float peaks[kSkinnyWaves][kSkinnyMaxM];
   const int tid = threadIdx.x, M = (int)a.M, K = (int)a.K;
   auto widen = [&](int m, int c, float* f) __attribute__((always_inline)) {  // values 8 c .. 8 c + 7 of row m
@@ -56,9 +66,9 @@ __device__ __forceinline__ void quantize_rows(const GemmArgs& a, uint8_t* codes,
       for (int c = tid; c < K / 8; c += T) {
         float f[8];
         widen(m, c, f);
-        *reinterpret_cast<uint2*>(codes + m * K + 8 * c) = encode8_group<DT, HN_KIND_INT8, ROUND>(f, peak, sc);
+        put(m * K + 8 * c, encode8_group<DT, HN_KIND_INT8, ROUND>(f, peak, sc));
       }
-      if (tid == 0) scales[m] = sc;
+      if (tid == 0) put_scale(m, sc);
     }
   } else {
     const int G = K / 128;
@@ -70,8 +80,8 @@ __device__ __forceinline__ void quantize_rows(const GemmArgs& a, uint8_t* codes,
 #pragma unroll
       for (int i = 0; i < 8; i++) peak = __builtin_fmaxf(peak, __builtin_fabsf(f[i]));
       peak = row16_max_nonneg(peak);
-      *reinterpret_cast<uint2*>(codes + m * K + (g * 16 + (tid & 15)) * 8) = encode8_group<DT, HN_KIND_INT8, ROUND>(f, peak, sc);
-      if ((tid & 15) == 0) scales[u] = sc;
+      put(m * K + (g * 16 + (tid & 15)) * 8, encode8_group<DT, HN_KIND_INT8, ROUND>(f, peak, sc));
+      if ((tid & 15) == 0) put_scale(u, sc);
     }
   }
   __syncthreads();

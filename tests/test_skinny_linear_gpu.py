@@ -77,3 +77,19 @@ def test_output_over_the_source(dev, layout, m, n, k, at):
         else:
             noalloc(src, w, sw, bias, group, "int8", out=out)
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("layout", ["g128", "channel", "block"])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (1, 300, 3072), (3, 130, 1152), (4, 64, 12288)])
+def test_workspace_holds_the_codes_and_scales(dev, layout, m, n, k):
+    from hy_nomas import _lib, kernels
+
+    x, w, sw, bias, group, sw_rows = linear_case(dev, layout, m, n, k)
+    ws = torch.full((_lib.lib().hn_block_linear_workspace_bytes(m, k, group),), 0x55, device=dev, dtype=torch.uint8)
+    out = torch.empty(m, n, dtype=x.dtype, device=dev)
+    entry(x, k, m, n, k, group, w, sw, sw_rows, bias, out, n, ws)
+    qa, sa = kernels.quantize_activations(x, group=group)
+    at = (m * k + 255) // 256 * 256
+    assert torch.equal(ws[:m * k].view(torch.int8).view(m, k), qa)
+    assert torch.equal(ws[at:at + sa.numel() * 4].view(torch.float32).view_as(sa), sa)
+    assert torch.equal(out, kernels.block_gemm(qa, sa, w, sw, bias, x.dtype))
