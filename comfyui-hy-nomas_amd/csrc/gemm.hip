@@ -169,7 +169,7 @@ static int launch_skinny_mode(GemmArgs& a, int epilogue, int out_dtype, hipStrea
   return launch_skinny_epi<4, MODE>(a, epilogue, out_dtype, st);
 }
 
-// The same from a 16-bit source (run_linear's M <= 4): codes and scales in LDS, outputs in the source's dtype.
+// The same from a 16-bit source (skinny_takes_source): codes and scales in LDS, outputs in the source's dtype.
 template <int MT, int MODE, int DT>
 static int launch_skinny_x(GemmArgs& a, int rounding, hipStream_t st) {
   constexpr int64_t ROWS = kSkinnyRows * kSkinnyWaves;
@@ -190,8 +190,9 @@ static int launch_skinny_x(GemmArgs& a, int rounding, hipStream_t st) {
 template <int MODE, int DT>
 static int launch_skinny_x_mode(GemmArgs& a, int rounding, hipStream_t st) {
   if (a.M == 1) return launch_skinny_x<1, MODE, DT>(a, rounding, st);
-  if (a.M == 2) return launch_skinny_x<2, MODE, DT>(a, rounding, st);
-  return launch_skinny_x<4, MODE, DT>(a, rounding, st);
+  if constexpr (MODE != 0)  // (skinny_takes_source: at most two rows there)
+    if (a.M > 2) return launch_skinny_x<4, MODE, DT>(a, rounding, st);
+  return launch_skinny_x<2, MODE, DT>(a, rounding, st);
 }
 
 template <int DT>
@@ -201,13 +202,28 @@ static int launch_skinny_x_dt(GemmArgs& a, bool g128, int rounding, hipStream_t 
   return launch_skinny_x_mode<1, DT>(a, rounding, st);
 }
 
-// Up to four rows whose codes fit 48 KB of LDS (three workgroups on a compute unit), 16-byte aligned, in a quantization
-// that the quantizer takes.  3072 -> 18432 at one row: 12.9 us, against 2.6 + 11.5 us for quantizer and GEMM.
-bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t group, int kind,
+// Whether the kernel that quantizes x itself takes a linear: 16-byte aligned 16-bit rows in a quantization that the quantizer
+// takes, where it was measured no slower than quantizer and GEMM.  Every workgroup (16 outputs wide) repeats the
+// quantization of all rows, so its cost grows with the rows, K and the workgroups that a compute unit runs, and past a point
+// exceeds the launch that it saves.  Times of the two launches over the one kernel's (graphs of calls over rotating
+// weights; worst of bf16 and fp16, 256 compute units), by K -> N:
+//   1 row    g128, blocks     1024 -> 512 1.44   3072 -> 18432 1.09   12288 -> 18432 1.02   3072 -> 36864 1.01   16384 -> 18432 0.97
+//            per token        1024 -> 512 1.37   3072 -> 18432 1.09   16384 -> 18432 1.07   3072 -> 36864 1.03
+//   2 rows   all              1024 -> 256 1.15   4096 -> 12288 1.04   6144 -> 12288 0.89    3072 -> 18432 0.90
+//            per token        8192 -> 4096 1.09  16384 -> 3072 1.08   8192 -> 18432 0.95
+//   3 rows   g128, blocks     1024 -> 4096 1.18  2048 -> 4096 1.11    4096 -> 5120 0.95     3072 -> 18432 0.87
+//   4 rows   g128, blocks     1024 -> 3072 1.18  3072 -> 3072 1.00    8192 -> 3072 0.87     12288 -> 18432 0.70
+//   3, 4 rows per token       1024 -> 512 1.03, 0.96                  3072 -> 18432 0.85, 0.78
+bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K, int64_t group, int kind,
                          int rounding, int out_dtype) {
-  return M > 0 && M <= kSkinnyMaxM && kind == HN_KIND_INT8 && (x_dtype == HN_DTYPE_BF16 || x_dtype == HN_DTYPE_F16) &&
-         out_dtype == x_dtype && M * K <= 49152 && (group == 128 || K <= 16384) && ldx >= K && ldx % 8 == 0 &&
-         ((uintptr_t)x & 15) == 0 && (rounding == HN_ROUND_HALF_AWAY || rounding == HN_ROUND_HALF_EVEN);
+  if (M <= 0 || M > kSkinnyMaxM || N <= 0 || kind != HN_KIND_INT8 || (x_dtype != HN_DTYPE_BF16 && x_dtype != HN_DTYPE_F16) ||
+      out_dtype != x_dtype || ldx < K || ldx % 8 || ((uintptr_t)x & 15) ||
+      (rounding != HN_ROUND_HALF_AWAY && rounding != HN_ROUND_HALF_EVEN))
+    return false;
+  const int64_t per_round = (int64_t)cu_count() * kSkinnyRows * kSkinnyWaves;  // outputs of one workgroup on each unit
+  if (M == 1) return K <= (group == 128 ? 12288 : 16384) && N <= 5 * per_round;
+  if (M == 2) return (K <= 4096 && N <= 3 * per_round) || (group != 128 && K <= 16384 && N <= per_round);
+  return group == 128 && K > 128 && M * K <= 8192 && N <= per_round;
 }
 
 // hn_block_gemm, or (x given, skinny_takes_source) the linear of x itself; qa [M, K] and sa [M, K / group] are then written.

@@ -429,7 +429,7 @@ int cu_count();  // compute units of the current device
 
 // The one-call linear (linear.hip): workspace size, argument checks, and quantize-then-GEMM into a
 // workspace that holds the activation codes and scales.
-bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, int64_t group, int kind,
+bool skinny_takes_source(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t N, int64_t K, int64_t group, int kind,
                          int rounding, int out_dtype);
 int skinny_linear(const void* x, int64_t ldx, int rounding, const void* qa, const float* sa, const void* qw, int64_t ldw,
                   const float* sw, int64_t ldsw, int64_t sw_rows, const void* bias, int bias_dtype, int64_t M, int64_t N,

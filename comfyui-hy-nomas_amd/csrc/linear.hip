@@ -41,7 +41,7 @@ int run_linear(const void* x, int x_dtype, int64_t ldx, int64_t M, int64_t K, in
   float* s = reinterpret_cast<float*>(ws + linear_scales_offset(M, K));
   const int64_t ng = K / group;
   const int64_t x_bytes = 2 * ((M - 1) * ldx + K);
-  if (skinny_takes_source(x, x_dtype, ldx, M, K, group, kind, rounding, out_dtype) &&
+  if (skinny_takes_source(x, x_dtype, ldx, M, N, K, group, kind, rounding, out_dtype) &&
       !overlap(x, x_bytes, out, 2 * ((M - 1) * ldo + N)) && !overlap(x, x_bytes, ws, linear_workspace_bytes(M, K, group)))
     return skinny_linear(x, ldx, rounding, ws, s, qw, ldw, sw, ldsw, sw_rows, bias, bias_dtype, M, N, K, group, out, out_dtype,
                          ldo, stream);

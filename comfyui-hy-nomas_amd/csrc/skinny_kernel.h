@@ -12,8 +12,8 @@
 //   * + bias (absent: -0.0), optional GELU, the same output conversion.
 //
 // With a source (SRC, the linear's 16-bit x) the kernel quantizes it itself: each workgroup forms the codes and scales
-// of its M rows in LDS, with the quantizer's own arithmetic, while its first weights are on the way.  At most 48 KB
-// of codes, read from L2 by every workgroup; in return the quantizer's launch and the codes' trip through memory go.  The
+// of its M rows in LDS, with the quantizer's own arithmetic, while its first weights are on the way.  At most 16 KB
+// of codes, from x read in L2 by every workgroup; in return the quantizer's launch and the codes' trip through memory go.  The
 // first workgroup also leaves them in a.qa and a.sa, the workspace where the linear's callers find them.
 #pragma once
 

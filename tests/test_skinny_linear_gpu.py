@@ -1,5 +1,5 @@
 """block_linear at M <= 4, where one kernel quantizes 16-bit rows itself, against the quantizer and the GEMM as separate
-calls: bit for bit, at the edges of its range (one group, odd widths, 48 KB of codes and one row past it)."""
+calls: bit for bit, at the edges of its range and past them (one group, odd widths, long rows)."""
 import pytest
 import torch
 
@@ -57,7 +57,7 @@ def linear_case(dev, layout, m, n, k, dt=torch.bfloat16):
 
 @pytest.mark.parametrize("layout", ["g128", "channel"])
 @pytest.mark.parametrize("m,n,k,at", [(1, 3072, 3072, 0), (4, 3072, 3072, 0), (4, 12288, 12288, 0), (2, 1000, 1152, 576),
-                                      (3, 6000, 8192, -64)])
+                                      (3, 4000, 2048, -64)])
 def test_output_over_the_source(dev, layout, m, n, k, at):
     """out in x's own rows, from column `at` on (before the first row: at < 0): every value of x is read before any output
     is stored, as with more rows, by either entry point."""
@@ -93,3 +93,36 @@ def test_workspace_holds_the_codes_and_scales(dev, layout, m, n, k):
     assert torch.equal(ws[:m * k].view(torch.int8).view(m, k), qa)
     assert torch.equal(ws[at:at + sa.numel() * 4].view(torch.float32).view_as(sa), sa)
     assert torch.equal(out, kernels.block_gemm(qa, sa, w, sw, bias, x.dtype))
+
+
+def launches(call):
+    """The kernels that a call records into a graph."""
+    import ctypes
+
+    from hy_nomas import _lib
+
+    call()
+    torch.cuda.synchronize()
+    graph, n = torch.cuda.CUDAGraph(keep_graph=True), ctypes.c_size_t()
+    with torch.cuda.graph(graph):
+        call()
+    assert _lib.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+# the largest sizes on 256 compute units at which one kernel was faster than quantizer and GEMM, and the next ones
+@pytest.mark.parametrize("layout,m,n,k,one", [
+    ("g128", 1, 18432, 3072, True), ("g128", 1, 64, 12288, True), ("block", 1, 64, 12416, False), ("g128", 1, 20488, 256, False),
+    ("channel", 1, 64, 16384, True), ("channel", 2, 12288, 512, True), ("channel", 2, 12296, 512, False),
+    ("g128", 2, 64, 4096, True), ("block", 2, 64, 4224, False), ("channel", 2, 4096, 16384, True), ("channel", 2, 4104, 4224, False), ("g128", 3, 4096, 256, True), ("g128", 3, 4104, 256, False),
+    ("block", 4, 64, 2048, True), ("g128", 4, 64, 2176, False), ("channel", 3, 64, 1024, False), ("g128", 4, 64, 128, False),
+    ("g128", 4, 18432, 12288, False)])
+def test_where_one_kernel_takes_the_linear(dev, layout, m, n, k, one):
+    from hy_nomas import kernels
+
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the sizes are for 256 compute units")
+    x, w, sw, bias, group, _ = linear_case(dev, layout, m, n, k)
+    assert launches(lambda: kernels.block_linear(x, w, sw, bias)) == (1 if one else 2)
+    qa, sa = kernels.quantize_activations(x, group=group)
+    assert torch.equal(kernels.block_linear(x, w, sw, bias), kernels.block_gemm(qa, sa, w, sw, bias, x.dtype))
