@@ -299,22 +299,24 @@ void attention_kernel(const AttnArgs a) {
     if (__builtin_amdgcn_ballot_w64(!(mrel + mref_m <= m + kSlack)) != 0) {
       const float mt = mrel + mref_m;
       const bool grow = mt > m + kSlack;
-      const float mnew = grow ? mt : m;
-      const float alpha = __builtin_amdgcn_exp2f(m - mnew);  // 1 where m stays, 0 for the first tile
-      m = mnew;
+      // where the reference stays nothing changes (m and m' differ only while every score so far was -inf: m = -inf and
+      // m' = 0, whose difference is no factor)
+      const float mnew = grow ? mt : mref_m;
+      const float alpha = grow ? __builtin_amdgcn_exp2f(m - mt) : 1.0f;  // 0 for the first tile
+      m = grow ? mt : m;
       lsum *= alpha;
 #pragma unroll
       for (int db = 0; db < 4; db++)
 #pragma unroll
         for (int r = 0; r < 16; r++) oacc[db][r] *= alpha;
       // this tile's scores moved to the new reference, and the next tiles' products start from it
-      const float delta = (mref_m - m) * inv_scale;
+      const float delta = (mref_m - mnew) * inv_scale;
 #pragma unroll
       for (int kb = 0; kb < 2; kb++)
 #pragma unroll
         for (int r = 0; r < 16; r++) s[kb][r] += delta;
-      mref_m = m;
-      const float mr = -m * inv_scale;
+      mref_m = mnew;
+      const float mr = -mnew * inv_scale;
 #pragma unroll
       for (int r = 0; r < 16; r++) mref[r] = mr;
     }

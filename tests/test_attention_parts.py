@@ -143,3 +143,25 @@ def test_argument_validation_without_a_gpu():
     assert lib.hn_segment_attention_workspace_bytes(_lib.int64s(part), 1, None, 0, 1, 1, 10) == 128 * 64 * 2
     assert lib.hn_segment_attention_workspace_bytes(_lib.int64s(part), 3, None, 0, 1, 1, 10) == -1
     assert ctypes.sizeof(_lib.int64s(part)) == 72
+
+
+# units (of 128 queries) x keys: the keys walked by one workgroup, and split into ranges that begin inside the mask
+@pytest.mark.gpu
+@pytest.mark.parametrize("h,lq,lk,masked", [(1, 129, 100, (0, 64)), (1, 129, 2000, (64, 1900)), (1, 129, 2000, (0, 1900)),
+                                            (2, 40, 1500, (700, 1500)), (24, 2700, 1500, (64, 1500))])
+def test_tiles_whose_scores_are_all_minus_infinity(dev, h, lq, lk, masked):
+    """Keys hidden from every other query by a product beyond the floats' range: whole tiles score -inf for some of a
+    wave's queries and not for others, first in a range of keys or later.  They take no weight."""
+    from hy_nomas import attention
+
+    q, k, v, _ = operands(dev, 1, h, max(lq, lk), 0, 0, lq + lk)
+    q, k, v = q[:, :lq].clone(), k[:, :lk].clone(), v[:, :lk]
+    q[..., 0] = 0
+    q[:, ::2, :, 0] = 4
+    k[:, masked[0]:masked[1], :, 0] = torch.finfo(torch.bfloat16).min
+    ref = ref_attention(q, k, v)
+    assert torch.isfinite(ref).all()
+    got = attention.attention(q, k, v, backend="hip")
+    assert torch.isfinite(got.float()).all()
+    fro, mx = rel(got, ref)
+    assert fro < 1e-2 and mx < 3e-2, (fro, mx)
