@@ -78,9 +78,10 @@ def values_buffer(b, h, lk, device, d=128):
 
 
 def _rows16(t):
-    """t with a contiguous last dim and 16-byte aligned rows (a copy only when needed)."""
+    """t with a contiguous last dim and 16-byte aligned rows (a copy only when needed).  The copy is a clone:
+    `contiguous()` returns a contiguous tensor as it is, also off a 16-byte boundary or with odd strides of size-1 dims."""
     if t.stride(-1) != 1 or t.data_ptr() % 16 or any(st % 8 for st in t.stride()[:-1]):
-        t = t.contiguous()
+        t = t.clone(memory_format=torch.contiguous_format)
     return t
 
 

@@ -165,3 +165,36 @@ def test_tiles_whose_scores_are_all_minus_infinity(dev, h, lq, lk, masked):
     assert torch.isfinite(got.float()).all()
     fro, mx = rel(got, ref)
     assert fro < 1e-2 and mx < 3e-2, (fro, mx)
+
+
+def off16(t, by=1):
+    """t's values in a contiguous tensor that starts `by` elements past a 16-byte boundary."""
+    flat = torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)[by:]
+    return flat.view(t.shape).copy_(t)
+
+
+def test_rows16_copies_what_contiguous_leaves():
+    """A contiguous tensor off a 16-byte boundary, and one whose size-1 dims have odd strides, are copied too."""
+    from hy_nomas import attention
+
+    t = torch.randn(1, 6, 2, 128).to(torch.bfloat16)
+    odd = torch.empty(3000, dtype=torch.bfloat16).as_strided((1, 6, 2, 128), (1537, 256, 128, 1)).copy_(t)
+    for x in (off16(t), off16(t, 4), odd, t[..., ::2].repeat_interleave(2, -1).transpose(2, 3).contiguous().transpose(2, 3)):
+        got = attention._rows16(x)
+        assert torch.equal(got, x) and got.stride(-1) == 1
+        assert got.data_ptr() % 16 == 0 and all(st % 8 == 0 for st in got.stride()[:-1])
+    assert attention._rows16(t) is t and attention._rows16(t[:, 1:]).data_ptr() == t[:, 1:].data_ptr()
+
+
+@pytest.mark.gpu
+def test_operands_off_the_16_byte_boundary(dev):
+    """Queries, keys, values and history that start anywhere, with and without groups: the aligned tensors' result."""
+    from hy_nomas import attention
+
+    q, k, v, hist = operands(dev, 1, 2, 130, 20, 70, 9)
+    for plan in (None, split_plan(dev, 130, 20, 2)):
+        want = attention.segment_attention(q, k, v, hist, plan, backend="hip")
+        got = attention.segment_attention(off16(q), off16(k, 2), off16(v), tuple(map(off16, hist)), plan, backend="hip")
+        assert torch.equal(got, want)
+    assert torch.equal(attention.attention(off16(q), off16(k), off16(v), backend="hip"),
+                       attention.attention(q, k, v, backend="hip"))
