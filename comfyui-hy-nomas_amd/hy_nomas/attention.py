@@ -188,6 +188,8 @@ def _attend_groups(q, k, v, hist, plan, out):
         # torch's own indexing of the row numbers: out-of-range rows are refused and negative ones counted from the
         # end, as indexing q, k and v themselves does
         rows = torch.arange(length, device=q.device)[idx]
+        if nq == 0:
+            continue  # nothing to write (nor, with no text either, a row to point to)
         groups, at_q, at_t = [], 0, 0
         for q_idx, text_idx in chunk:
             groups.append((at_q, q_idx.numel(), at_t, text_idx.numel()))

@@ -198,3 +198,22 @@ def test_operands_off_the_16_byte_boundary(dev):
         assert torch.equal(got, want)
     assert torch.equal(attention.attention(off16(q), off16(k), off16(v), backend="hip"),
                        attention.attention(q, k, v, backend="hip"))
+
+
+@pytest.mark.gpu
+def test_groups_without_queries(dev):
+    """Plans whose groups, all of them or those of a whole launch (past the 64th), name no query or text rows."""
+    from hy_nomas import attention
+
+    q, k, v, hist = operands(dev, 1, 2, 70, 6, 40, 11)
+    none, text = torch.arange(0, device=dev), torch.arange(2, device=dev)
+    rows = torch.arange(50, device=dev)
+    for groups in ([(none, none)], [(none, text)], [(rows, text)] + [(none, none)] * 64, [(none, none)] * 70 + [(rows, text)]):
+        out = torch.zeros_like(q)
+        attention._segment(q, k, v, hist, Plan(70, groups), "hip", out=out)
+        assert (out[:, 50:] == 0).all()
+        if any(t.numel() for t, _ in groups):
+            fro, mx = rel(out[:, :50], per_group(q, k, v, hist, Plan(70, [(rows, text)]))[:, :50])
+            assert fro < 1e-2 and mx < 3e-2, (fro, mx)
+        else:
+            assert (out == 0).all()
