@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import oracle
-from conftest import seeded
+from conftest import recorded_kernels, seeded
 from test_gemm_gpu import int8_weights
 from test_quant_gpu import outlier_input
 
@@ -101,3 +101,27 @@ def test_mid_tile_rows_equal_the_small_tiles(dev, layout, m, n, k):
             full = kernels.block_gemm(qa, sa, w, sw, bias, dt, kind, epi)
             part = kernels.block_gemm(qa[rows].contiguous(), sa_rows, w, sw, bias, dt, kind, epi)
             assert torch.equal(full[rows], part), (dt, epi)
+
+
+# (workgroups, threads) on 256 compute units: a ring tile's or the persistent tiles'
+@pytest.mark.parametrize("layout,m,n,k,kernel", [
+    ("g128", 64, 16384, 256, (256, 256)), ("g128", 100, 5000, 384, (158, 256)), ("channel", 300, 10888, 256, (430, 256)),
+    # one round of 128 x 128 tiles: a ring of eight waves, for int8 g128 the two-stage tile of four
+    ("channel", 300, 8200, 256, (195, 512)), ("fp8", 300, 8200, 256, (195, 512)), ("g128", 300, 8200, 256, (195, 256)),
+    # two rounds of 128 x 64, for fp8 up to K = 8192
+    ("g128", 300, 12000, 256, (470, 256)), ("fp8", 300, 12000, 8192, (470, 256)), ("fp8", 300, 12000, 8320, (282, 256))])
+def test_which_tile_serves_a_problem(dev, layout, m, n, k, kernel):
+    from hy_nomas import kernels
+
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the sizes are for 256 compute units")
+    kind = "fp8" if layout == "fp8" else "int8"
+    x = torch.randn(m, k, generator=seeded(k), dtype=torch.float32).to(torch.bfloat16).to(dev)
+    qa, sa = kernels.quantize_activations(x, kind, None if layout == "channel" else 128)
+    w = torch.randint(-100, 100, (n, k), dtype=torch.int8, device=dev)
+    w = (w.float() / 50).to(torch.float8_e4m3fn) if kind == "fp8" else w
+    sw = torch.full(((n + 127) // 128 if kind == "fp8" else n, 1 if layout == "channel" else k // 128), 1e-3, device=dev)
+    kernels.validate_scales(sw)
+    assert recorded_kernels(lambda: kernels.block_gemm(qa, sa, w, sw, kind=kind)) == [kernel]
+    assert torch.equal(kernels.block_gemm(qa, sa, w, sw, kind=kind),
+                       kernels.block_gemm(qa, sa, w, sw, None, torch.float32, kind=kind).to(torch.bfloat16))

@@ -3,7 +3,7 @@ calls: bit for bit, at the edges of its range and past them (one group, odd widt
 import pytest
 import torch
 
-from conftest import seeded
+from conftest import recorded_kernels, seeded
 from test_gemm_gpu import int8_weights
 
 pytestmark = pytest.mark.gpu
@@ -95,21 +95,6 @@ def test_workspace_holds_the_codes_and_scales(dev, layout, m, n, k):
     assert torch.equal(out, kernels.block_gemm(qa, sa, w, sw, bias, x.dtype))
 
 
-def launches(call):
-    """The kernels that a call records into a graph."""
-    import ctypes
-
-    from hy_nomas import _lib
-
-    call()
-    torch.cuda.synchronize()
-    graph, n = torch.cuda.CUDAGraph(keep_graph=True), ctypes.c_size_t()
-    with torch.cuda.graph(graph):
-        call()
-    assert _lib.lib().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
-    return n.value
-
-
 # the largest sizes on 256 compute units at which one kernel was faster than quantizer and GEMM, and the next ones
 @pytest.mark.parametrize("layout,m,n,k,one", [
     ("g128", 1, 18432, 3072, True), ("g128", 1, 64, 12288, True), ("block", 1, 64, 12416, False), ("g128", 1, 20488, 256, False),
@@ -123,6 +108,6 @@ def test_where_one_kernel_takes_the_linear(dev, layout, m, n, k, one):
     if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
         pytest.skip("the sizes are for 256 compute units")
     x, w, sw, bias, group, _ = linear_case(dev, layout, m, n, k)
-    assert launches(lambda: kernels.block_linear(x, w, sw, bias)) == (1 if one else 2)
+    assert len(recorded_kernels(lambda: kernels.block_linear(x, w, sw, bias))) == (1 if one else 2)
     qa, sa = kernels.quantize_activations(x, group=group)
     assert torch.equal(kernels.block_linear(x, w, sw, bias), kernels.block_gemm(qa, sa, w, sw, bias, x.dtype))
