@@ -217,3 +217,81 @@ def test_groups_without_queries(dev):
             assert fro < 1e-2 and mx < 3e-2, (fro, mx)
         else:
             assert (out == 0).all()
+
+
+# few queries over many keys (split), and several blocks over few (not)
+@pytest.mark.gpu
+@pytest.mark.parametrize("lv,lt,lh", [(129, 40, 1900), (300, 130, 60)])
+def test_non_finite_operands(dev, lv, lt, lh):
+    """Infinite and NaN values reach the outputs that weigh them, a NaN query only its own row, and a key of infinite
+    scores takes no weight (-inf) or makes its query NaN (+inf), through the packed values and the joined partials."""
+    from hy_nomas import attention
+
+    q, k, v, hist = operands(dev, 1, 2, lv, lt, lh, 17)
+    plan = split_plan(dev, lv, lt, 2)
+    hist[1][0, 3, 0, 5], v[0, 70, 0, 6], v[0, lv + 1, 1, 7] = float("inf"), float("-inf"), float("nan")
+    q[0, 9, 1, 0], k[0, 2, 1, 3] = float("nan"), float("inf")
+    got, ref = attention.segment_attention(q, k, v, hist, plan, backend="hip").float(), per_group(q, k, v, hist, plan)
+    assert torch.equal(got.isnan(), ref.isnan()) and ref.isnan().any() and (~ref.isnan()).any()
+    assert torch.equal(got.isinf(), ref.isinf()) and torch.equal(got[got.isinf()], ref[ref.isinf()])
+    fin = ref.isfinite()
+    fro, mx = rel(got[fin], ref[fin])
+    assert fro < 1e-2 and mx < 3e-2, (fro, mx)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("h,lv,lt,lh", [(2, 129, 40, 1900), (24, 2700, 100, 300)])
+def test_repeated_calls_give_the_same_bits(dev, h, lv, lt, lh):
+    from hy_nomas import attention
+
+    q, k, v, hist = operands(dev, 1, h, lv, lt, lh, 23)
+    for plan in (None, split_plan(dev, lv, lt, 3)):
+        first = attention.segment_attention(q, k, v, hist, plan, backend="hip")
+        for _ in range(3):
+            assert torch.equal(attention.segment_attention(q, k, v, hist, plan, backend="hip"), first)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("groups", [0, 3])
+def test_segment_attention_under_graph_capture(dev, groups):
+    """One captured call replayed on fresh inputs, with eager work and synchronizations between the replays."""
+    from hy_nomas import attention
+
+    lv, lt, lh = 129, 40, 1900
+    q, k, v, hist = operands(dev, 1, 2, lv, lt, lh, 29)
+    plan = split_plan(dev, lv, lt, groups) if groups else None
+
+    def call():
+        return attention.segment_attention(q, k, v, hist, plan, backend="hip")
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    torch.cuda.synchronize()
+    for replay in range(3):
+        for t, new in zip((q, k, v, *hist), (*(x := operands(dev, 1, 2, lv, lt, lh, 31 + replay))[:3], *x[3])):
+            t.copy_(new)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, call()), replay
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,h,lq,lk", [(1, 1, 1, 1), (2, 3, 200, 130), (1, 2, 129, 2000), (1, 24, 2700, 400)])
+def test_entry_point_without_a_workspace(dev, b, h, lq, lk):
+    """hn_attention, whose query blocks are never split, against float32."""
+    from hy_nomas import _lib, attention
+
+    q, k, v, _ = operands(dev, b, h, max(lq, lk), 0, 0, lq * lk)
+    q, k, v, out = q[:, :lq], k[:, :lk], v[:, :lk], torch.empty(b, lq, h, 128, dtype=torch.bfloat16, device=dev)
+    vt = attention.transpose_values(v.transpose(1, 2))
+    _lib.call("hn_attention", *attention._operand(q), *attention._operand(k), vt.data_ptr(), *vt.stride()[:3],
+              *attention._operand(out), b, h, lq, lk, 128, 128 ** -0.5, _lib.stream(q))
+    fro, mx = rel(out, ref_attention(q, k, v))
+    assert fro < 1e-2 and mx < 3e-2, (fro, mx)

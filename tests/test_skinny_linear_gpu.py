@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [(1, 15, 128), (1, 1000, 3072), (2, 257, 384), (3, 130, 16384), (4, 64, 12288), (4, 48, 16384),
                                    (4, 333, 1152)])
 def test_equals_quantizer_then_gemm(dev, layout, m, n, k):
-    from hy_nomas import kernels
+    from hy_nomas import _lib, kernels
 
     print(f"skinny linear {layout} m={m} n={n} k={k}", flush=True)
     w, sw, bias = int8_weights(n, k, n + k, layout == "channel")
@@ -32,9 +32,13 @@ def test_equals_quantizer_then_gemm(dev, layout, m, n, k):
             want = kernels.block_gemm(qa, sa, w.to(dev), sw.to(dev), b, dt)
             got = kernels.block_linear(xd, w.to(dev), sw.to(dev), b, rounding=rounding)
             assert torch.equal(got, want), (dt, rounding)
-            wide = torch.zeros(m, k + 64, dtype=dt, device=dev)
+            # rows of a wider source (block_linear copies those, the entry point reads them where they lie)
+            wide = torch.full((m, k + 64), float("nan"), dtype=dt, device=dev)
             wide[:, :k] = xd
-            assert torch.equal(kernels.block_linear(wide[:, :k], w.to(dev), sw.to(dev), b, rounding=rounding), want)
+            group, out = k if layout == "channel" else 128, torch.empty_like(want)
+            ws = torch.empty(_lib.lib().hn_block_linear_workspace_bytes(m, k, group), device=dev, dtype=torch.uint8)
+            entry(wide, k + 64, m, n, k, group, w.to(dev), sw.to(dev), 128 if layout == "block" else 1, b, out, n, ws, rounding)
+            assert torch.equal(out, want)
 
 
 def entry(x, ldx, m, n, k, group, w, sw, sw_rows, bias, out, ldo, ws, rounding="half_away"):
@@ -53,6 +57,26 @@ def linear_case(dev, layout, m, n, k, dt=torch.bfloat16):
     x = torch.randn(m, k, generator=seeded(m + k)).to(dt).to(dev)
     return (x, w.to(dev), sw.to(dev), bias.to(dt).to(dev), k if layout == "channel" else 128,
             128 if layout == "block" else 1)
+
+
+@pytest.mark.parametrize("layout", ["g128", "channel", "block"])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_infinities_and_nan_in_the_source(dev, layout, dt):
+    """Their rows (or groups) take the scales and codes, bit for bit, that the quantizer gives them."""
+    from hy_nomas import _lib, kernels
+
+    m, n, k = 2, 130, 1152
+    x, w, sw, bias, group, sw_rows = linear_case(dev, layout, m, n, k, dt)
+    x[0, 5], x[0, 300], x[0, 400], x[1, 700:828] = float("inf"), float("-inf"), float("nan"), float("nan")
+    ws = torch.empty(_lib.lib().hn_block_linear_workspace_bytes(m, k, group), device=dev, dtype=torch.uint8)
+    for rounding in ("half_away", "half_even"):
+        out = torch.empty(m, n, dtype=dt, device=dev)
+        entry(x, k, m, n, k, group, w, sw, sw_rows, bias, out, n, ws, rounding)
+        qa, sa = kernels.quantize_activations(x, group=group, rounding=rounding)
+        at = (m * k + 255) // 256 * 256
+        assert torch.equal(ws[:m * k].view(torch.int8).view(m, k), qa)
+        assert torch.equal(ws[at:at + sa.numel() * 4].view(torch.int32), sa.view(torch.int32).flatten())
+        assert torch.equal(out.view(torch.int16), kernels.block_gemm(qa, sa, w, sw, bias, dt).view(torch.int16))
 
 
 @pytest.mark.parametrize("layout", ["g128", "channel"])
