@@ -32,13 +32,15 @@
 // query's group.  Every segment starts a new 64-key tile, and its last tile is masked, so nothing is joined in
 // memory first; V^T holds the segments one after another, each padded to whole tiles (attention_pack_kernel).  All
 // groups share one launch, which fills the chip where one group would not.  Joining, gathering and transposing per
-// group took two thirds of such a call: 24 heads, 3520 + 200 tokens over 15840 history keys in three groups went
-// from 2595 to 941 us; 16 heads x 26656 tokens, where only the V^T pass is new, from 5777 to 5448 us.
+// group took two thirds of such a call.  With the split keys below, 24 heads, 3520 + 200 tokens over 15840 history keys in
+// three groups went from 2608 to 905 us; 16 heads x 26656 tokens, where the V^T pass and the split are new, from 5649 to
+// 4995 us.
 //
 // Lazy rescale.  The running reference max m moves only when a tile's max exceeds it by more than 8 (base-2
 // units), so the probabilities exp2(s - m) stay below 2^8 and the accumulators are rescaled only a few times
 // per query instead of whenever the max grows.  The result is the same quotient: numerator and denominator
 // share the reference.
+// A query whose scores so far are all -inf has no reference yet: m = -inf, and its products start from 0.
 #include "hn_common.h"
 
 namespace hn {
@@ -434,7 +436,7 @@ __global__ __launch_bounds__(kCombineThreads) void attention_combine_kernel(cons
 // each of the 128 V^T rows, keys past the segment's end as zeros.  HBM bound: 2 bytes read and 2 written per
 // element.  Text keys are gathered by row on the way (a few hundred rows at most), and their K rows copied to the
 // packed buffer, where the attention kernel's tile loads can take them as a segment.  46 us for 24 heads x 19600
-// keys, 5.2 TB/s; torch's permuting copy of one such V took about 400 us.
+// keys, 5.3 TB/s; torch's permuting copy of one such V took about 400 us.
 struct PackPart {
   const uint16_t* v;
   int64_t svb, svh, svj;

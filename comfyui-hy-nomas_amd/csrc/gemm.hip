@@ -21,8 +21,8 @@ enum class TileSplit { kBig, kMid, kSmall, kBoth };
 // tiles; when the last round would leave more than half of the compute units idle, its rows go to 128 x 128
 // tiles (four per big tile, on every compute unit).  A problem with fewer big tiles than half a round runs on
 // small tiles alone, and one whose bn x 192 tiles still fit one round takes those: the round is shorter (256 x 192
-// against 256 x 256 tiles, us, g128 / per token / fp8 blocks: 3520 x 12288 -> 3072 218 / 146 / 163 -> 191 / 135 / 148,
-// 3520 x 3072 -> 3072 64.8 / 39.7 / 48.8 -> 55.6 / 34.4 / 41.3, 5000 x 8192 -> 2048 143 / 96 / 107 -> 128 / 90 / 99).  With
+// against 256 x 256 tiles, us, g128 / per token / fp8 blocks: 3520 x 12288 -> 3072 227 / 129 / 138 -> 190 / 120 / 131,
+// 3520 x 3072 -> 3072 55.5 / 38.4 / 41.1 -> 50.2 / 35.2 / 37.1, 5000 x 8192 -> 2048 130 / 84 / 96 -> 118 / 79 / 89).  With
 // more rounds than one they lose what they gain: a round of them takes 0.9 of the big tile's for 0.75 of its work.
 static TileSplit choose_tiles(int64_t M, int64_t N, int bm, int bn, int64_t slots, int64_t* big_rows) {
   const int64_t tm = (M + bm - 1) / bm, tn = (N + bn - 1) / bn, tiles = tm * tn;
@@ -68,8 +68,8 @@ static int launch_group(GemmArgs& a, bool g128, hipStream_t st) {
   constexpr bool SWIGLU = EPI == HN_EPI_SWIGLU_QUANT;
   constexpr bool SMALL_OK = EPI == HN_EPI_NONE || EPI == HN_EPI_GELU;
   // epilogues that need a token's 128 channels in one wave: four waves of 128 x 32 where the problem would fill at
-  // most half of the compute units with the big tile (200 x 3072 -> 9216 q/k/v heads 52 -> 25 us g128, 32 -> 19 per
-  // token; -> 12288 GELU + requantization 73 -> 28)
+  // most half of the compute units with the big tile (200 x 3072 -> 9216 q/k/v heads 64 -> 32 us g128, 49 -> 28 per
+  // token; -> 12288 GELU + requantization 68 -> 32 and 54 -> 30)
   constexpr bool WAVE_ROWS = KIND == HN_KIND_INT8 && (EPI == HN_EPI_GELU_QUANT || EPI == kEpiQkvHeads);
   constexpr int ESZ = OUT_DT == HN_DTYPE_F32 ? 4 : 2;
   if (!g128) {

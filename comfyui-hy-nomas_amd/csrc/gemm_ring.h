@@ -18,8 +18,8 @@ namespace hn {
 enum class RingTile { kNone, k64x32, k64x64, k128x64, k128x128 };  // channels x tokens
 
 // The smallest tile that covers the problem in one round of workgroups; 128 x 64 also serves two per compute unit,
-// where it fills the chip better than 128 x 128 tiles that no longer fit one round (300 x 2048 -> 12288: 23.2 -> 18.2
-// us g128, 15.8 -> 13.1 per token).  Larger problems keep the persistent tiles: from two full rounds of 128 x 128 on
+// where it fills the chip better than 128 x 128 tiles that no longer fit one round (300 x 2048 -> 12288: 25.8 -> 22.1
+// us g128, 20.1 -> 17.4 per token).  Larger problems keep the persistent tiles: from two full rounds of 128 x 128 on
 // those move fewer bytes per product (1024 x 3072 -> 12288: 72 us against 85).  So do, over random sizes of the class:
 //   int8 g128 where only 128 x 128 tiles fit one round: that ring took 0.89 to 1.14 of the two-stage tile's time, 1.04 at
 //     the median (844 x 2816 -> 3584 19.8 against 22.2 us, 605 x 3840 -> 6400 32.6 against 36.7); 128 x 64 two to a
@@ -28,11 +28,11 @@ enum class RingTile { kNone, k64x32, k64x64, k128x64, k128x128 };  // channels x
 //     0.69 to 1.00 of it up to 8192.
 // GEMM alone, old and new (us):
 //   tokens x K -> N        int8 g128        int8 per token   fp8 blocks
-//   32 x 12288 -> 3072     85.7 -> 39.1     76.5 -> 24.7     80.8 -> 30.4
-//   100 x 3072 -> 3072     21.6 -> 10.9     19.4 -> 7.5      20.2 -> 9.2
-//   200 x 12288 -> 3072    88.9 -> 43.6     76.4 -> 26.9     83.1 -> 32.6
-//   500 x 3072 -> 3072     23.0 -> 17.0     19.9 -> 11.5     21.1 -> 13.4
-//   1024 x 3072 -> 3072    24.7             20.7 -> 15.1     22.1 -> 18.4
+//   32 x 12288 -> 3072     92.8 -> 44.4     85.1 -> 28.3     90.7 -> 32.3
+//   100 x 3072 -> 3072     27.1 -> 11.1     24.8 -> 9.4      26.5 -> 10.2
+//   200 x 12288 -> 3072    94.5 -> 36.1     84.0 -> 29.3     91.0 -> 32.1
+//   500 x 3072 -> 3072     26.9 -> 19.8     24.1 -> 15.0     25.6 -> 16.8
+//   1024 x 3072 -> 3072    23.4             20.3 -> 16.1     21.6 -> 18.6
 template <int KIND, bool G128>
 inline RingTile choose_ring(int64_t M, int64_t N, int64_t K) {
   const int64_t cus = cu_count();

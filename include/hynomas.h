@@ -189,7 +189,9 @@ int hn_attention(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const voi
 /*
  * hn_attention with a workspace (16-byte aligned, hn_attention_workspace_bytes, which may be 0), in which several
  * workgroups can share a query block's keys where the queries alone would leave the chip idle: each leaves an fp32
- * partial output with its maximum and sum, and a second pass joins them.
+ * partial output with its maximum and sum, and a second pass joins them.  Which query blocks are shared, and over how
+ * many workgroups, depends on B, H, Lq, Lk and the device's compute units, and with it the rounding of a query's result
+ * (the same call always gives the same bits).  hn_attention never shares: a query's result depends on its keys alone.
  */
 int64_t hn_attention_workspace_bytes(int64_t B, int64_t H, int64_t Lq, int64_t Lk);
 int hn_attention_ws(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const void* k, int64_t skb, int64_t skh,
@@ -209,7 +211,8 @@ int hn_attention_ws(const void* q, int64_t sqb, int64_t sqh, int64_t sqi, const 
  * A group's queries attend to all parts, then to the group's text rows.  A query row in several groups takes the
  * last one's result; a row in none is not written.  bf16, D == 128, strides in elements, rows 16-byte aligned
  * (out 8-byte), token strides of k and v in (0, 2^23]; B * H <= 65535.  The workspace (256-byte aligned) holds V^T,
- * the gathered text keys and the partials of split keys (hn_attention_ws): hn_segment_attention_workspace_bytes, which returns -1 for bad counts.
+ * the gathered text keys and the partials of split keys (hn_attention_ws): hn_segment_attention_workspace_bytes, which
+ * returns -1 for bad counts.
  */
 int64_t hn_segment_attention_workspace_bytes(const int64_t* parts, int n_parts, const int64_t* groups, int n_groups,
                                              int64_t B, int64_t H, int64_t Lq);
